@@ -44,6 +44,23 @@ def test_router_logits_exact(dev, m, e, h, xdt, wdt):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("m,e,h,xdt,wdt,skew", [
+    (5, 1, 32, "bf16", "f32", 0), (16, 17, 64, "f32", "bf16", 0), (17, 256, 544, "bf16", "bf16", 0),
+    (65, 40, 96, "f32", "f32", 0), (273, 256, 64, "bf16", "f32", 0), (530, 250, 96, "bf16", "f32", 0),
+    (33, 24, 64, "bf16", "f32", 1)])
+def test_router_logits_matrix_tiles(dev, m, e, h, xdt, wdt, skew):
+    """Edges of the fp64 matrix kernel's token and expert tiles, one chunk of h and fewer chunks than
+    waves, each of its three tile plans; skew: rows that are not 16-byte aligned (the other kernel)."""
+    from mosaic_amd import ops
+    rng = np.random.default_rng(m + e + h)
+    dt = {"bf16": torch.bfloat16, "f32": torch.float32}
+    x = torch.from_numpy(rng.standard_normal((m, h)).astype(np.float32)).to(dt[xdt])
+    w = torch.from_numpy((rng.standard_normal((e, h)) * 0.02).astype(np.float32)).to(dt[wdt])
+    xd = torch.empty(m * h + skew, dtype=x.dtype, device=dev)[skew:].view(m, h).copy_(x)
+    got = ops.router_logits(xd, w.to(dev)).cpu().numpy()
+    np.testing.assert_array_equal(got, MO.router_logits(x.float().numpy(), w.float().numpy()))
+
+
 def _v4_cfg(e=256, h=1024, k=8):
     return SimpleNamespace(n_routed_experts=e, hidden_size=h, scoring_func="sqrtsoftplus", num_experts_per_tok=k,
                            norm_topk_prob=True, routed_scaling_factor=1.5)
