@@ -963,6 +963,11 @@ __device__ __forceinline__ void mla_copy16(const void* g, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
                "v"(g) : "memory", "m0");
 }
+// the same from a wave-uniform base plus this lane's byte offset
+__device__ __forceinline__ void mla_copy16_s(const void* base, int off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
+               "v"(off), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void mla_copy4(const void* g, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds)),
                "v"(g) : "memory", "m0");
@@ -1476,6 +1481,422 @@ __global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const uint16_t* 
     out[((int64_t)b * H + 16 * ht + 4 * hq + r) * kMlaDl + 16 * dt + (lane & 15)] = f32_bf16(acc[r]);
 }
 
+// Sparse attention of many query rows (a prompt) over a bf16 cache of 512-wide
+// rows (V = K).  An item is one (row, group of 16 HT heads); its whole pick
+// list goes through one workgroup and the normalized output is written
+// directly, so there are no partials and no combine.  At most one workgroup of
+// eight waves a CU walks the items w, w + grid, ...
+//
+// An item's valid picks are compacted first (order kept), so masked picks cost
+// nothing and only the last block's tail is masked.  Blocks of 32 picks move
+// through a ring of four LDS stages by global -> LDS copies (one 1 KB row an
+// instruction), issued three blocks ahead by the value waves.  Waves 0..3 score
+// block p (wave w: head tile w, q in registers; K rows from LDS) and soft-max it
+// into P, while waves 4..7 multiply block p - 1 (wave 4 + w: columns 128 w ..
+// + 127 of every head tile, V read out of the K rows with transposing reads), so
+// each SIMD holds one wave of either kind and the two contractions, the
+// softmax chain and the LDS reads overlap.  The first K fragments of a block
+// and all its V fragments are read in the period before their products.  One
+// barrier a period hands over the stage, P and the rescale factors.  Both
+// products have the picks' or columns' side as their MFMA rows, so a lane's
+// entries share a head.
+//
+// The items' blocks form one sequence: the next item's picks are loaded at the
+// start of an item and compacted during it, its first blocks are copied during
+// the last three periods, its q is prefetched, and the value waves normalize and
+// store an item while the scoring waves are in the next one.  An item takes at
+// least kMrMinPeriods periods (the compaction's hand-overs).
+//
+// Bound by the chains of a period (scoring: 32 MFMAs on LDS operands, then the
+// softmax; value: copies, then 32 MFMAs) and by the gather, 32 KB a block and
+// CU: 2048 rows x 64 heads x 512 with 128 + up to 512 picks 686 -> 185 us
+// (550 TFLOP/s on the valid picks), of which copies alone take ~100.
+constexpr int kMrStages = 4;
+constexpr int kMrRow = kMlaDl * 2 + 16;  // bytes per staged row
+constexpr int kMrStage = kMlaBT * kMrRow;
+constexpr int kMrMaxPicks = 2048;
+constexpr int kMrMinRows = 64;
+constexpr int kMrCopies = kMlaBT / 4;  // copies a value wave a block
+constexpr int kMrMinPeriods = 8;
+constexpr int kMrPer = kMrMaxPicks / 512;  // picks a thread
+constexpr float kLog2e = 1.4426950408889634f;
+
+template <int HT>
+__global__ void __launch_bounds__(512) mla_rows_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
+                                                       const int32_t* __restrict__ idx, const float* __restrict__ sink,
+                                                       uint16_t* __restrict__ out, int64_t n, int rows,
+                                                       int rows_per_kv, int n_groups, int topk, float scale) {
+  constexpr int NSQ = kMlaDl / 32, DTW = kMlaDt / 4;
+  constexpr int KS = kMrRow / 2;
+  __shared__ __attribute__((aligned(16))) uint8_t Kt[kMrStages * kMrStage];
+  __shared__ __attribute__((aligned(16))) uint16_t Ps[2][16 * HT * kPsStride];
+  __shared__ float As[2][16 * HT], Ml[2][16 * HT];
+  __shared__ int Fl[2][HT];
+  __shared__ int Ids[2][kMrMaxPicks];
+  __shared__ int cnt[kMrPer][8];
+  __shared__ float Sink[256];  // heads <= 256
+  const int H = HT * 16 * n_groups;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, qd = lane >> 4;
+  const int n_items = rows * n_groups;
+  // item -> row (a prompt's last rows have the most picks: first) and head group
+  auto row_of = [&](int it) { return rows - 1 - it / n_groups; };
+  int idv[kMrPer], before[kMrPer];
+  auto load_picks = [&](int it) {
+    const int64_t r0 = (int64_t)row_of(it) * topk;
+#pragma unroll
+    for (int k = 0; k < kMrPer; ++k) {
+      const int t = 512 * k + tid;
+      idv[k] = t < topk ? idx[r0 + t] : -1;
+    }
+  };
+  // compaction, first half: each wave's valid picks counted
+  auto count_picks = [&]() {
+#pragma unroll
+    for (int k = 0; k < kMrPer; ++k) {
+      const bool ok = idv[k] >= 0 && (int64_t)idv[k] < n;
+      if (!ok) idv[k] = -1;
+      const uint64_t mask = __ballot(ok);
+      before[k] = __popcll(mask & ((1ull << lane) - 1));
+      if (lane == 0) cnt[k][wv] = __popcll(mask);
+    }
+  };
+  // second half, a barrier later: the picks into `dst` in order; returns their number
+  auto place_picks = [&](int* dst) {
+    int nv = 0;
+#pragma unroll
+    for (int k = 0; k < kMrPer; ++k)
+#pragma unroll
+      for (int w = 0; w < 8; ++w) {
+        if (w == wv && idv[k] >= 0) dst[nv + before[k]] = idv[k];
+        nv += cnt[k][w];
+      }
+    return __builtin_amdgcn_readfirstlane(nv);
+  };
+  auto blocks_of = [&](int nv) { return (nv + kMlaBT - 1) / kMlaBT; };
+  int it = blockIdx.x;  // grid <= n_items
+  load_picks(it);
+  if (sink && tid < H) Sink[tid] = sink[tid];
+  count_picks();
+  __syncthreads();
+  int nv = place_picks(Ids[0]), nv_next = 0;
+  __syncthreads();
+  int par = 0;     // picks buffer of the current item
+  int stage = 0;   // ring stage of the item's next block (the period's block p)
+  int period = 0;  // parity of P, the factors and the flags
+  // copies of block j of an item into a stage: rows 4 wv + i; slots past the
+  // last pick repeat its row (masked in the softmax).  The wave's picks are read
+  // ahead (lane i: row i), so an issue waits for no LDS round trip.
+  auto read_ids = [&](const int* ids, int nvj, int j) {
+    return ids[max(0, min(j * kMlaBT + kMrCopies * (wv & 3) + (lane & (kMrCopies - 1)), nvj - 1))];
+  };
+  auto issue = [&](int ids4, const uint16_t* base, int stg, int i) {
+    mla_copy16_s(base + (int64_t)__builtin_amdgcn_readlane(ids4, i) * kMlaDl, 16 * lane,
+                 mla_lds_addr(&Kt[(stg % kMrStages) * kMrStage + (kMrCopies * (wv - 4) + i) * kMrRow]));
+  };
+  auto cache_of = [&](int i) { return kv + (int64_t)(row_of(i) / rows_per_kv) * n * kMlaDl; };
+  // every copy of this wave but those of this period has landed, then the
+  // barrier (a value wave's stores of an item are its period's last, and may fly)
+  constexpr int kStores = HT * DTW / 2;
+  auto hand_over = [&](bool flying, bool stored) {
+    if (wv < 4)
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else if (flying && stored)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMrCopies + kStores) : "memory");
+    else if (stored)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kStores) : "memory");
+    else if (flying)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kMrCopies) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  const uint16_t* kvb = cache_of(it);  // the item's cache, and the next one's (set once an item: divisions)
+  const uint16_t* kvn = kvb;
+  for (int j = 0; j < (wv < 4 ? 0 : min(3, blocks_of(nv))); ++j) {
+    const int ids4 = read_ids(Ids[0], nv, j);
+#pragma unroll
+    for (int i = 0; i < kMrCopies; ++i) issue(ids4, kvb, j, i);
+  }
+  int id4 = read_ids(Ids[0], nv, 3);  // the picks of the next block to copy
+  // One period's shared work at period p of the item: the next item's picks, and
+  // the copies three blocks ahead (of this item, or the next one's first three),
+  // set up here and issued by copy().
+  bool cp_on = false;
+  const uint16_t* cp_base = nullptr;
+  int cp_ids = 0, cp_stage = 0;
+  auto advance = [&](int p, int nblk, int nper, int next) {
+    if (next < n_items) {
+      if (p == 2) count_picks();
+      if (p == 3) nv_next = place_picks(Ids[par ^ 1]);
+    }
+    if (wv < 4) return;
+    const int j = p + 3 - nper;  // block of the next item (nper >= 8: its picks were placed a barrier ago)
+    const bool own = p + 3 < nblk;
+    cp_on = own || (j >= 0 && next < n_items && j < blocks_of(nv_next));
+    cp_ids = id4;
+    cp_base = own ? kvb : kvn;
+    // (the stages the current item has left count from its end)
+    cp_stage = own ? stage + 3 : stage + (nblk > p ? nblk - p : 0) + j;
+    // next period: block p + 4 of this item, or block j + 1 of the next
+    id4 = j + 1 >= 0 ? read_ids(Ids[par ^ 1], nv_next, j + 1) : read_ids(Ids[par], nv, p + 4);
+  };
+  auto copy = [&]() {
+    if (!cp_on) return;
+#pragma unroll
+    for (int i = 0; i < kMrCopies; ++i) issue(cp_ids, cp_base, cp_stage, i);
+  };
+  if (wv < 4) {
+    const bool scorer = wv < HT;
+    bf16x8_t qn[NSQ];
+    auto load_q = [&](int i) {
+      const uint16_t* qrow =
+          q + ((int64_t)row_of(i) * H + 16 * ((i % n_groups) * HT + (scorer ? wv : 0)) + c) * kMlaDl;
+#pragma unroll
+      for (int s = 0; s < NSQ; ++s) qn[s] = *reinterpret_cast<const bf16x8_t*>(qrow + 32 * s + 8 * qd);
+    };
+    load_q(it);
+    // S^T tiles: rows = slots 16 j + 4 qd + r, column = head c, so a lane's scores
+    // share a head: its running maximum, and this lane's part of the sum
+    const float sl2 = scale * kLog2e;  // probabilities as exp2(s * scale * log2(e) - m)
+    int krow[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) krow[j] = mla_slot_token(16 * j + c) * KS + 8 * qd;
+    // K fragments in batches of KB steps, read two batches ahead of the products;
+    // the first two of a block are read at the end of the period before
+    constexpr int KB = 2, NKB = NSQ / KB;
+    bf16x8_t kop[3][KB][2];
+    auto read_k = [&](int stg, int kb2, bf16x8_t (&dst)[KB][2]) {
+      const uint16_t* kst = reinterpret_cast<const uint16_t*>(&Kt[(stg % kMrStages) * kMrStage]);
+#pragma unroll
+      for (int ss = 0; ss < KB; ++ss)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          dst[ss][j] = *reinterpret_cast<const bf16x8_t*>(&kst[krow[j] + 32 * (kb2 * KB + ss)]);
+    };
+    hand_over(false, false);
+    if (scorer && nv > 0) {
+      read_k(0, 0, kop[0]);
+      read_k(0, 1, kop[1]);
+    }
+    for (; it < n_items;) {
+      const int next = it + gridDim.x;
+      const int nblk = blocks_of(nv), nper = max(nblk, kMrMinPeriods);
+      bf16x8_t qb[NSQ];
+#pragma unroll
+      for (int s = 0; s < NSQ; ++s) {
+        qb[s] = qn[s];
+        asm volatile("" : "+v"(qb[s]));
+      }
+      kvn = cache_of(min(next, n_items - 1));
+      load_picks(min(next, n_items - 1));
+      load_q(min(next, n_items - 1));
+      float m_run = -INFINITY, l_run = 0.f;
+      for (int p = 0; p < nper; ++p) {
+        advance(p, nblk, nper, next);
+        const bool score = scorer && p < nblk;
+        f32x4_t st[2], st2[2];
+        if (score) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) st[j] = st2[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb2 = 0; kb2 < NKB; ++kb2) {
+            if (kb2 + 2 < NKB) read_k(stage, kb2 + 2, kop[(kb2 + 2) % 3]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ss = 0; ss < KB; ++ss)
+#pragma unroll
+              for (int j = 0; j < 2; ++j) {
+                const int s = kb2 * KB + ss;
+                if (s & 1)
+                  st2[j] = mfma_bf16(kop[kb2 % 3][ss][j], qb[s], st2[j]);
+                else
+                  st[j] = mfma_bf16(kop[kb2 % 3][ss][j], qb[s], st[j]);
+              }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        // next period's block (this item's, or the next one's first) has landed
+        if (scorer && (p + 1 < nblk || (p + 1 == nper && next < n_items && nv_next > 0))) {
+          read_k(stage + (p < nblk ? 1 : 0), 0, kop[0]);
+          read_k(stage + (p < nblk ? 1 : 0), 1, kop[1]);
+        }
+        if (score) {
+          float sv[2][4];
+          bool over = false;  // the running maximum moves only past the lazy margin (or from -inf)
+          const float lim = m_run + kMlaLazyMax * kLog2e;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            st[j] += st2[j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sv[j][r] = st[j][r] * sl2;
+          }
+          if ((p + 1) * kMlaBT > nv) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                sv[j][r] = p * kMlaBT + mla_slot_token(16 * j + 4 * qd + r) < nv ? sv[j][r] : -INFINITY;
+          }
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) over |= sv[j][r] > lim;
+          const bool move = __ballot(over) != 0;
+          if (move) {  // rare past the first block
+            float bm = -INFINITY;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) bm = fmaxf(bm, sv[j][r]);
+            bm = fmaxf(bm, __shfl_xor(bm, 16));
+            bm = fmaxf(bm, __shfl_xor(bm, 32));
+            const float m_new = bm > lim ? bm : m_run;
+            const float alpha = (bm > lim && m_run != -INFINITY) ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+            l_run *= alpha;
+            m_run = m_new;
+            if (qd == 0) As[period & 1][16 * wv + c] = alpha;
+          }
+          if (lane == 0) Fl[period & 1][wv] = move ? 1 : 0;
+          uint16_t* ps = Ps[period & 1];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            float pr[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              pr[r] = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sv[j][r] - m_run);
+              l_run += pr[r];
+            }
+            const uint2 pw = {__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{pr[0], pr[1]}, bf16x2_t)),
+                              __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{pr[2], pr[3]}, bf16x2_t))};
+            *reinterpret_cast<uint2*>(&ps[(16 * wv + c) * kPsStride + 16 * j + 4 * qd]) = pw;
+          }
+        }
+        if (scorer && p == nper - 1) {  // the item's maxima and sums, read by the value waves next period
+          float l = l_run;
+          l += __shfl_xor(l, 16);
+          l += __shfl_xor(l, 32);
+          if (qd == 0) {
+            Ml[0][16 * wv + c] = m_run;
+            Ml[1][16 * wv + c] = l;
+          }
+        }
+        hand_over(false, false);
+        stage += p < nblk ? 1 : 0;
+        ++period;
+      }
+      it = next;
+      par ^= 1;
+      nv = nv_next;
+      kvb = kvn;
+    }
+    return;
+  }
+  // value waves: O^T tiles, rows = columns 16 (dt0 + dl) + 4 qd + r, column = head 16 ht + c
+  const int dt0 = (wv - 4) * DTW;
+  f32x4_t o[HT][DTW];
+#pragma unroll
+  for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+    for (int dl = 0; dl < DTW; ++dl) o[ht][dl] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int vi = c >> 2, vj = c & 3;
+  // multiply the block scored last period (parity pb), whose V fragments were
+  // read during that period, and read those of the block scored in this one
+  bf16x8_t vv[DTW];
+  auto read_v = [&](int stg, int dd) {
+    const uint16_t* vp = reinterpret_cast<const uint16_t*>(&Kt[(stg % kMrStages) * kMrStage]) +
+                         (8 * qd + 2 * vi) * KS + 4 * vj + 16 * (dt0 + dd);
+    const mla_v4s a = lds_read_tr16(vp), e = lds_read_tr16(vp + KS);
+    return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, e, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto value = [&](int stg, int pb) {
+    int fl[HT];
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) fl[ht] = Fl[pb][ht];
+    bf16x8_t pa[HT];
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht)
+      pa[ht] = *reinterpret_cast<const bf16x8_t*>(&Ps[pb][(16 * ht + c) * kPsStride + 8 * qd]);
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+      if (__builtin_amdgcn_readfirstlane(fl[ht])) {  // the same word for every lane
+        const float al = As[pb][16 * ht + c];
+#pragma unroll
+        for (int dl = 0; dl < DTW; ++dl) o[ht][dl] *= al;
+      }
+    }
+#pragma unroll
+    for (int dd = 0; dd < DTW; ++dd) {
+#pragma unroll
+      for (int ht = 0; ht < HT; ++ht) o[ht][dd] = mfma_bf16(vv[dd], pa[ht], o[ht][dd]);
+      __builtin_amdgcn_sched_barrier(0);
+      vv[dd] = read_v(stg, dd);  // (unused if no block is scored in this period)
+    }
+  };
+  // normalize and store an item, and clear the tiles for the next
+  auto store = [&](int i) {
+    const int64_t b = row_of(i);
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+      const int head = 16 * ((i % n_groups) * HT + ht) + c;
+      const float m = Ml[0][16 * ht + c];
+      const float l =
+          Ml[1][16 * ht + c] + ((sink && m != -INFINITY) ? __builtin_amdgcn_exp2f(Sink[head] * kLog2e - m) : 0.f);
+      const float inv = m == -INFINITY ? 0.f : 1.0f / l;
+      // two column tiles at a time: lane rows 4 qd .. + 3 of both are exchanged
+      // (row 1 of the first with row 0 of the second, 3 with 2), so that a lane
+      // stores 8 consecutive columns: tile dl + (qd & 1), columns 8 (qd >> 1) ..
+      uint16_t* orow = out + (b * H + head) * kMlaDl + 16 * (dt0 + (qd & 1)) + 8 * (qd >> 1);
+#pragma unroll
+      for (int dl = 0; dl < DTW; dl += 2) {
+        uint32_t w[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x4_t v = o[ht][dl + t] * inv;
+          o[ht][dl + t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          w[t][0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[0], v[1]}, bf16x2_t));
+          w[t][1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[2], v[3]}, bf16x2_t));
+        }
+        const auto x0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto x1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        *reinterpret_cast<u32x4_t*>(orow + 16 * dl) = u32x4_t{x0[0], x1[0], x0[1], x1[1]};
+      }
+    }
+  };
+  hand_over(false, false);
+  bool scored = false;  // a block was scored last period
+  int prev = -1;        // the item to store
+  for (; it < n_items;) {
+    const int next = it + gridDim.x;
+    const int nblk = blocks_of(nv), nper = max(nblk, kMrMinPeriods);
+    kvn = cache_of(min(next, n_items - 1));
+    load_picks(min(next, n_items - 1));
+    for (int p = 0; p < nper; ++p) {
+      advance(p, nblk, nper, next);
+      if (scored) {
+        value(stage, (period - 1) & 1);
+      } else if (p < nblk) {
+#pragma unroll
+        for (int dd = 0; dd < DTW; ++dd) vv[dd] = read_v(stage, dd);
+      }
+      copy();
+      const bool stored = p == 0 && prev >= 0;
+      if (stored) store(prev);
+      hand_over(cp_on, stored);
+      scored = p < nblk;
+      stage += scored ? 1 : 0;
+      ++period;
+    }
+    prev = it;
+    it = next;
+    par ^= 1;
+    nv = nv_next;
+    kvb = kvn;
+  }
+  if (scored) value(stage, (period - 1) & 1);
+  store(prev);
+}
+
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct IndexerWs {
@@ -1808,6 +2229,27 @@ extern "C" int mosaic_mla_sparse_decode_bf16(const uint16_t* q, const uint16_t* 
   int rc = check_mla_common(rows, h, n, topk, rows_per_kv, workspace, workspace_bytes);
   if (rc) return rc;
   if (rows == 0) return kOk;
+  // From 64 rows the row kernel: splitting a row over workgroups no longer pays
+  // for its partials and combine (64 heads, us, split path against rows: 32 rows
+  // of 640 picks 27.1 / 32.3, 64 rows 40.1 / 33.6, 64 rows of 2048 picks 86.1 /
+  // 82.5, 128 rows 112.7 / 83.7; 16 heads, 64 rows of 640 30.6 / 24.6).
+  if (d == 512 && topk <= kMrMaxPicks && rows >= kMrMinRows) {
+    int ht = 4;
+    while (ht > 1 && (h / 16) % ht != 0) --ht;
+    const int groups = (int)(h / (16 * ht));
+    const dim3 grid((unsigned)std::min<int64_t>(rows * groups, 256));
+    hipStream_t st = (hipStream_t)stream;
+    switch (ht) {
+#define MLA_CASE(HTV)                                                                                                  \
+  case HTV:                                                                                                            \
+    MOSAIC_LAUNCH((mla_rows_kernel<HTV>), grid, dim3(512), 0, st, q, kv, idx, sink, out, n, (int)rows,                 \
+                  (int)rows_per_kv, groups, (int)topk, softmax_scale);                                                 \
+    break;
+      MLA_CASE(1) MLA_CASE(2) MLA_CASE(3) MLA_CASE(4)
+#undef MLA_CASE
+    }
+    MOSAIC_RETURN_LAUNCH("mla_rows");
+  }
   const MlaKv kvd{kv, nullptr, nullptr, n, (int)rows_per_kv, 0};
   if (d == 576)
     return launch_mla<false, 64>(q, kvd, sink, idx, out, rows, h, topk, softmax_scale, workspace, (hipStream_t)stream);

@@ -282,6 +282,32 @@ def test_mla_bf16_kv_vs_oracle(dev, d, rows, h, n, t):
     _close(out.float().cpu().numpy(), D.sparse_attn(q, kv, sink, idx, d ** -0.5, 512, rows // nb))
 
 
+@pytest.mark.parametrize("rows,h,n,t,per_kv,masked", [
+    (64, 64, 300, 1, 64, 0.0), (64, 16, 40, 33, 32, 0.0), (70, 48, 500, 257, 70, 0.5), (300, 32, 700, 64, 150, 0.9),
+    (129, 128, 900, 600, 129, 0.3), (65, 64, 2100, 2048, 65, 0.0), (520, 64, 90, 31, 260, 0.95)])
+def test_mla_rows_bf16_vs_oracle(dev, rows, h, n, t, per_kv, masked):
+    """The one-pass row kernel (64 rows and more): one and many items a workgroup, rows without a valid
+    pick and with a few (fewer blocks than its pipeline's periods), tails of a 32-pick block, picks
+    masked in the middle or past the cache, every head-tile count, and rows whose running maximum moves."""
+    from mosaic_amd import ops
+    rng = np.random.default_rng(rows + t)
+    q = C.round_bf16(rng.standard_normal((rows, h, 512)).astype(np.float32))
+    kv = C.round_bf16(rng.standard_normal((rows // per_kv, n, 512)).astype(np.float32))
+    idx = rng.integers(0, n, (rows, t)).astype(np.int32)
+    idx[rng.random(idx.shape) < masked] = -1
+    idx[0] = -1
+    idx[rows // 2, : t // 2] = n + 5
+    sink = rng.standard_normal(h).astype(np.float32)
+    scale = 512 ** -0.5 if rows != 70 else 0.4
+    T = lambda a: torch.from_numpy(a).to(dev)
+    out = ops.mla_sparse_decode_bf16(T(q).to(torch.bfloat16), T(kv).to(torch.bfloat16), T(idx), scale, T(sink))
+    # a sample of the rows: both ends, the masked one, and some between
+    pick = sorted({0, 1, rows // 2, rows - 1, *rng.integers(0, rows, 8).tolist()})
+    for r in pick:
+        ref = D.sparse_attn(q[r:r + 1], kv[r // per_kv][None], sink, idx[r:r + 1], scale, 512, 1)
+        _close(out[r:r + 1].float().cpu().numpy(), ref)
+
+
 def test_upstream_sparse_attn_signature(dev):
     """sparse_attn(q [b,m,h,d], kv [b,n,d], sink, idx [b,m,t], scale), h < 16 padded (inference_kernel.py:355-368)."""
     from mosaic_amd.kernels.dsa import sparse_attn, sparse_attn_fused
