@@ -929,6 +929,262 @@ __global__ void __launch_bounds__(1024) dsa_finish_kernel(const uint64_t* __rest
   }
 }
 
+// ---------------------------------------------- many rows over short caches
+// Indexer + exact top-k of many query rows that share short key caches (a
+// prompt: row t sees the first (t + 1) / ratio entries).  Picks are most of a
+// row's entries there, so bounding first would save little: every entry gets
+// its exact score, and the row's keys are sorted, in one kernel without a
+// workspace.
+//
+// A workgroup takes kDrRows consecutive rows of one cache, one wave each (q's
+// int8 limbs in registers).  The cache goes through LDS in chunks of 128 tokens,
+// already as int8 limbs in MFMA operand order (wave w converts tokens 16 w ..
+// + 15 of a chunk for all the rows), the next chunk's codes loaded during the
+// products.  Row i of the A operand holds head (i / 4) * H / 4 + 4 j + i % 4 in
+// head tile j, so lane quarter qd holds the terms of heads qd H / 4 .. + H / 4 - 1
+// of token c, and the canonical head order is four runs of in-lane additions
+// with the sum handed from quarter to quarter.  The five limb sums go through
+// two int32 before one fp64 multiply-add (|g0 + 2^7 g1| and |g2 + 2^7 g3 + 2^14
+// g4| < 2^30).  Then each wave sorts its row: a bitonic network over E keys a lane.
+//
+// Bound by the matrix unit and the term arithmetic about equally (1152 MFMA
+// cycles and ~1400 VALU cycles a wave per 16 tokens and row).
+constexpr int kDrRows = 8;
+constexpr int kDrMaxL = 2048;
+constexpr int kDrChunk = 128;
+
+// Sort keys as positive doubles in [1, 2): the mantissa holds the 32-bit score
+// key, then kDrIdxBits of the inverted token.  Their order is the keys', and a
+// compare-exchange is one v_max_f64 and one v_min_f64 (no NaN, infinity or
+// subnormal among them).
+constexpr int kDrIdxBits = 11;
+static_assert(kDrMaxL <= 1 << kDrIdxBits, "a token must fit its bits of the key");
+__device__ __forceinline__ double key_max(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double key_min(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double key_flip(double a, uint32_t sign) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, a);
+  return __builtin_bit_cast(double, u ^ ((uint64_t)sign << 32));
+}
+
+// Descending bitonic sort over the wave, position lane * E + e.  The lanes whose
+// runs a phase sorts upwards hold their keys negated during it, so every
+// exchange keeps the larger key at the lower position.
+template <int E>
+__device__ __forceinline__ void wave_sort_desc(double (&x)[E]) {
+  const int lane = threadIdx.x & 63;
+  auto order = [&](double& a, double& b) {
+    const double t = key_max(a, b);
+    b = key_min(a, b);
+    a = t;
+  };
+  // runs of E in each lane, descending in even lanes
+#pragma unroll
+  for (int sz = 2; sz < E; sz *= 2)
+#pragma unroll
+    for (int st = sz / 2; st > 0; st /= 2)
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (!(e & st)) {
+          if ((e & sz) == 0)
+            order(x[e], x[e | st]);
+          else
+            order(x[e | st], x[e]);
+        }
+  uint32_t up = 0u;  // sign of this lane's keys in the current phase
+  auto phase = [&](bool desc) {
+    const uint32_t want = desc ? 0u : 0x80000000u;
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = key_flip(x[e], want ^ up);
+    up = want;
+  };
+  auto merge = [&]() {
+#pragma unroll
+    for (int st = E / 2; st > 0; st /= 2)
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (!(e & st)) order(x[e], x[e | st]);
+  };
+  phase((lane & 1) == 0);
+  merge();
+  for (int sz = 2; sz <= 64; sz *= 2) {
+    phase((lane & sz) == 0);  // (the last size: all descending)
+    for (int st = sz / 2; st > 0; st /= 2) {
+      double y[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) y[e] = __shfl_xor(x[e], st);
+      if (lane & st) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = key_min(x[e], y[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = key_max(x[e], y[e]);
+      }
+    }
+    merge();
+  }
+}
+
+// sort the n <= 64 E scores of a row and write its topk picks; `buf` is the
+// row's LDS (its scores, then its sorted indices)
+template <int E>
+__device__ __forceinline__ void dsa_row_picks(float* buf, int n, int topk, int offset, int32_t* dst) {
+  const int lane = threadIdx.x & 63;
+  constexpr uint32_t kMask = (1u << kDrIdxBits) - 1;
+  double x[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int t = 64 * e + lane;
+    // (a token's inverted bits are never 0 past the last one, so no key equals the padding's)
+    const uint64_t key = ((uint64_t)key_low_nan(buf[t]) << kDrIdxBits) | (uint64_t)(kMask - (uint32_t)t);
+    x[e] = __builtin_bit_cast(double, 0x3FF0000000000000ull | (t < n ? key + 1 : 0ull));
+  }
+  wave_sort_desc<E>(x);
+  wave_lds_fence();
+  int* sorted = reinterpret_cast<int*>(buf);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    sorted[lane * E + e] = (int)(kMask - ((uint32_t)(__builtin_bit_cast(uint64_t, x[e]) - 1) & kMask));
+  wave_lds_fence();
+  const int kk = min(topk, n);
+  for (int i = lane; i < topk; i += 64) dst[i] = i < kk ? sorted[i] + offset : -1;
+}
+
+template <int HT>
+__global__ void __launch_bounds__(64 * kDrRows) dsa_rows_topk_kernel(
+    const uint8_t* __restrict__ q, const float* __restrict__ qs, const uint8_t* __restrict__ k,
+    const float* __restrict__ ks, const float* __restrict__ w, const int32_t* __restrict__ lengths,
+    int32_t* __restrict__ idx_out, int64_t L, int groups, int kdiv, int64_t kstride, int topk, int offset) {
+  constexpr int H = HT * 16, HB = H / 4;
+  __shared__ i32x4_v kls[kDrChunk / 16][2][3][64];
+  __shared__ float kss[kDrChunk];
+  __shared__ float scs[kDrRows][kDrMaxL];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int c = lane & 15, qd = lane >> 4;
+  // a cache's last rows first: in a prompt they see the most entries
+  const int g = (int)blockIdx.x % groups, r0 = ((kdiv + kDrRows - 1) / kDrRows - 1 - (int)blockIdx.x / groups) * kDrRows;
+  const bool active = r0 + wv < kdiv;
+  const int64_t row = (int64_t)g * kdiv + (active ? r0 + wv : r0);
+  const int n = active ? (int)row_length(lengths, (int)row, L) : 0;
+  int nmax = 0;
+  for (int r = r0; r < min(r0 + kDrRows, kdiv); ++r)
+    nmax = max(nmax, (int)row_length(lengths, g * kdiv + r, L));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  const uint8_t* kb = k + (int64_t)g * kstride * kIdxD;
+  const float* ksb = ks + (int64_t)g * kstride;
+  u32x4_t kx[2];
+  float kscale = 0.f;
+  auto load_chunk = [&](int t0) {
+    const int t = t0 + 16 * wv + c;
+    const bool ok = t < L;
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch)
+      kx[ch] = ok ? *reinterpret_cast<const u32x4_t*>(kb + (int64_t)t * kIdxD + 64 * ch + 16 * qd) : u32x4_t{0u, 0u, 0u, 0u};
+    kscale = ok ? ksb[t] : 0.f;
+  };
+  if (nmax > 0) load_chunk(0);
+  i32x4_v ql[HT][2][3];
+  float qsv[HT][4], wvv[HT][4];
+#pragma unroll
+  for (int j = 0; j < HT; ++j) {
+    const uint8_t* qrow = q + (row * H + (c >> 2) * HB + 4 * j + (c & 3)) * kIdxD + 16 * qd;
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) e4m3_limbs(*reinterpret_cast<const u32x4_t*>(qrow + 64 * ch), ql[j][ch]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      qsv[j][r] = qs[row * H + qd * HB + 4 * j + r];
+      wvv[j][r] = w[row * H + qd * HB + 4 * j + r];
+    }
+  }
+  for (int t0 = 0; t0 < nmax; t0 += kDrChunk) {
+    __syncthreads();  // the previous chunk is no longer read
+    {
+      i32x4_v o[2][3];
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch) {
+        e4m3_limbs(kx[ch], o[ch]);
+#pragma unroll
+        for (int la = 0; la < 3; ++la) kls[wv][ch][la][lane] = o[ch][la];
+      }
+      if (qd == 0) kss[16 * wv + c] = kscale;
+    }
+    __syncthreads();
+    if (t0 + kDrChunk < nmax) load_chunk(t0 + kDrChunk);
+    const int nb = min(kDrChunk / 16, (n - t0 + 15) / 16);  // batches of this row in the chunk (<= 0: none)
+    for (int bt = 0; bt < nb; ++bt) {
+      i32x4_v kl[2][3];
+#pragma unroll
+      for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+        for (int la = 0; la < 3; ++la) kl[ch][la] = kls[bt][ch][la][lane];
+      const float ksc = kss[16 * bt + c];
+      float tv[HB];
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        i32x4_v gs[5];
+#pragma unroll
+        for (int mm = 0; mm < 5; ++mm) gs[mm] = i32x4_v{0, 0, 0, 0};
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+          for (int la = 0; la < 3; ++la)
+#pragma unroll
+            for (int lb = 0; lb < 3; ++lb) gs[la + lb] = mfma_i8(ql[j][ch][la], kl[ch][lb], gs[la + lb]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int x0 = (gs[1][r] << 7) + gs[0][r];
+          const int x1 = (gs[4][r] << 14) + ((gs[3][r] << 7) + gs[2][r]);
+          // x1 2^14 + x0 is 2^18 times the exact dot, and exact in fp64
+          const float d = (float)fma((double)x1, 16384.0, (double)x0) * 0x1p-18f;
+          const float a = (d * qsv[j][r]) * ksc;
+          const float rr = a > 0.f ? a : 0.f;
+          tv[4 * j + r] = rr * wvv[j][r];
+        }
+      }
+      // heads in order: quarter 0's, then 1's, ... (each quarter's lanes go on from the previous one's sum)
+      float sum = 0.f;
+#pragma unroll
+      for (int h = 0; h < HB; ++h) sum = sum + tv[h];
+      sum = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false)[0]);
+#pragma unroll
+      for (int h = 0; h < HB; ++h) sum = sum + tv[h];
+      {
+        const uint32_t odd = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false)[1];
+        sum = __uint_as_float(__builtin_amdgcn_permlane32_swap(odd, odd, false, false)[0]);
+      }
+#pragma unroll
+      for (int h = 0; h < HB; ++h) sum = sum + tv[h];
+      sum = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false)[0]);
+#pragma unroll
+      for (int h = 0; h < HB; ++h) sum = sum + tv[h];
+      if (qd == 3) scs[wv][t0 + 16 * bt + c] = sum;
+    }
+  }
+  wave_lds_fence();
+  if (!active) return;
+  int32_t* dst = idx_out + row * topk;
+  if (n <= 64)
+    dsa_row_picks<1>(scs[wv], n, topk, offset, dst);
+  else if (n <= 128)
+    dsa_row_picks<2>(scs[wv], n, topk, offset, dst);
+  else if (n <= 256)
+    dsa_row_picks<4>(scs[wv], n, topk, offset, dst);
+  else if (n <= 512)
+    dsa_row_picks<8>(scs[wv], n, topk, offset, dst);
+  else if (n <= 1024)
+    dsa_row_picks<16>(scs[wv], n, topk, offset, dst);
+  else
+    dsa_row_picks<32>(scs[wv], n, topk, offset, dst);
+}
+
 // ===================================================================== MLA
 constexpr int kMlaBT = 32;        // tokens per online-softmax block
 constexpr int kMlaDl = 512;       // latent (value) width
@@ -2089,6 +2345,28 @@ static int indexer_topk_impl(const uint8_t* q, const float* q_s, const uint8_t* 
                    workspace_bytes, need);
   if (b == 0) return kOk;
   hipStream_t st = (hipStream_t)stream;
+  // The row kernel: on the shortest caches, and where many rows share a short
+  // one (us, certified path against row kernel, 64 heads: 1 row of 64 tokens 19.2
+  // / 13.0; 256 rows sharing 128 tokens 28.0 / 24.0, 256 tokens 34.0 / 40.1; 512
+  // rows sharing 256 tokens 52.8 / 40.9, 512 tokens 75.5 / 71.5, 1024 tokens 117 /
+  // 136; 1024 rows sharing 1024 tokens 180 / 140; 4096 rows sharing 1024 tokens
+  // 617 / 281).  A row takes one wave, so few rows over a longer cache, or rows
+  // with a cache each, leave it to the certified path.
+  if (l > 0 && (l <= 64 || (kdiv >= kDrRows && b >= 256 && (l <= 128 || (b >= 512 && l <= b && l <= kDrMaxL))))) {
+    const int groups = (int)(b / kdiv);
+    const dim3 grid((unsigned)(groups * ((kdiv + kDrRows - 1) / kDrRows)));
+#define MOSAIC_ROWS_TOPK(HT)                                                                                        \
+  MOSAIC_LAUNCH((dsa_rows_topk_kernel<HT>), grid, dim3(64 * kDrRows), 0, st, q, q_s, k, k_s, w, lengths, idx_out, l, \
+                groups, (int)kdiv, kstride, (int)topk, (int)offset)
+    switch (h / 16) {
+      case 1: MOSAIC_ROWS_TOPK(1); break;
+      case 2: MOSAIC_ROWS_TOPK(2); break;
+      case 3: MOSAIC_ROWS_TOPK(3); break;
+      default: MOSAIC_ROWS_TOPK(4); break;
+    }
+#undef MOSAIC_ROWS_TOPK
+    MOSAIC_RETURN_LAUNCH("dsa_indexer_topk_rows");
+  }
   IndexerWs ws;
   indexer_ws(b, l, (char*)workspace, &ws);
   const int64_t qwords = b * h * (kIdxD / 4);

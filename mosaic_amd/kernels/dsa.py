@@ -201,8 +201,9 @@ class Indexer(torch.nn.Module):
         q2 = q_fp8.reshape(bsz * seqlen, h, d)
         qs2, w2 = q_scale.reshape(bsz * seqlen, h).float(), weights.reshape(bsz * seqlen, h).float()
         if start_pos == 0:  # causal: position i scores the first (i + 1) // ratio compressed entries
-            bounds = (torch.arange(1, seqlen + 1, device=q_fp8.device) // ratio).to(torch.int32)
-            lengths = bounds.repeat(bsz)
+            lengths = torch.arange(1, seqlen + 1, device=q_fp8.device, dtype=torch.int32) // ratio
+            if bsz > 1:
+                lengths = lengths.repeat(bsz)
         else:
             lengths = torch.full((bsz * seqlen,), n_c, dtype=torch.int32, device=q_fp8.device)
         # the caches are read in place (their first n_c tokens, cache length = the buffer's)

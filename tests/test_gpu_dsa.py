@@ -391,6 +391,36 @@ def test_indexer_drop_in_decode(dev):
     np.testing.assert_array_equal(got.reshape(bsz, 512), ref)
 
 
+@pytest.mark.parametrize("groups,rows,h,l,cache,topk,ties", [
+    (1, 1, 64, 1, 1, 1, 0), (1, 3, 16, 16, 16, 5, 0), (5, 5, 48, 64, 70, 512, 1), (2, 256, 32, 17, 40, 2048, 0),
+    (1, 256, 64, 128, 128, 100, 1), (2, 514, 64, 129, 129, 64, 0), (1, 600, 64, 300, 333, 512, 1),
+    (1, 520, 64, 513, 520, 512, 0), (1, 1030, 16, 1025, 1025, 2048, 1), (1, 2048, 16, 2048, 2048, 700, 1)])
+def test_indexer_rows_kernel_vs_oracle(dev, groups, rows, h, l, cache, topk, ties):
+    """Rows over short caches in one kernel: every sort width, batches of 16 and chunks of 128 tokens cut
+    short, workgroups with idle waves, caches longer than l, lengths below 0, past l and 0, equal scores,
+    and NaN scores (lowest)."""
+    from mosaic_amd import ops
+    rng = np.random.default_rng(rows + l)
+    q, qs = D.quantize_rows_e4m3(rng.standard_normal((rows, h, 128)))
+    k, ks = D.quantize_rows_e4m3(rng.standard_normal((groups, cache, 128)))
+    w = rng.standard_normal((rows, h)).astype(np.float32)
+    if ties:
+        k[:, 1::3] = k[:, :1]
+        ks[:, 1::3] = ks[:, :1]
+        ks[:, 5 % cache] = np.nan
+    lengths = rng.integers(0, l + 1, rows).astype(np.int32)
+    lengths[0], lengths[-1], lengths[rows // 2] = l, l + 9, -1
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    kd, ksd = T(k)[:, :l], T(ks)[:, :l]
+    got = ops.dsa_indexer_topk_shared(T(q), T(qs), kd, ksd, T(w), topk, T(lengths), 3).cpu().numpy()
+    per = rows // groups
+    for r in sorted({0, rows - 1, rows // 2, *rng.integers(0, rows, 12).tolist()}):
+        g = r // per
+        ref = D.indexer_topk(q[r:r + 1], qs[r:r + 1], k[g:g + 1, :l], ks[g:g + 1, :l], w[r:r + 1], topk,
+                             np.clip(lengths[r:r + 1], 0, l), 3)
+        np.testing.assert_array_equal(got[r:r + 1], ref)
+
+
 def test_indexer_drop_in_prefill_causal(dev):
     """Indexer scoring at start_pos 0: position i sees the first (i + 1) // 4
     compressed entries, masked picks are -1, valid ones + offset (the query
