@@ -1059,34 +1059,43 @@ __global__ void __launch_bounds__(256) mx_gemm_a8_reduce_kernel(const float* __r
   *reinterpret_cast<uint2*>(y + i) = o;
 }
 
-// The dense plan: the staged kernel holds one workgroup per CU (160 KB of LDS),
-// so a plan aims at one round of at most 256 workgroups.  Up to 256 rows the
-// tiles are mostly 64 rows (the light loop streams the weight at the full per-CU rate
-// and the row tiles of a weight slice share it in L2); above, 256 rows (the
-// full loop does four times the MFMAs per staged weight byte).  K is split
-// while the tiles cover at most half of the CUs, at most 8 ways and into whole
-// 512-K chunks; the weight is then re-read by fewer workgroups than rows would
-// need.  Small-M plans keep the row tiles of one weight slice on one XCD (row
-// tile fastest), large-M plans the column tiles of one activation slice.
-static DenseA8Plan dense_a8_plan_tr(int64_t m, int64_t n, int64_t k, int tr) {
-  DenseA8Plan p;
-  p.tr = tr;
-  p.n_row = (int)((m + p.tr - 1) / p.tr);
-  p.n_col = (int)((n + 255) / 256);
-  const int tiles = p.n_row * p.n_col, nch = (int)(k / 512);
-  p.splits = 1;
-  if (tiles * 2 <= 256) p.splits = std::max(1, std::min({8, nch, 256 / tiles}));
-  p.row_fastest = p.tr == 64 ? 1 : 0;
-  return p;
+// The dense plan: tiles of 64 rows (the light loop, which streams the weight at
+// the full per-CU rate; the row tiles of a weight slice share it in L2, so they
+// are walked row tile fastest) or 256 rows (four times the MFMAs per staged
+// weight byte), and a split of K into up to 8 slices of whole 512-K chunks, by
+// the least estimated time.  The kernel holds one workgroup per CU (160 KB of
+// LDS), so a plan runs in rounds of 256 workgroups of (fixed + steps) time, plus
+// the split's partials written, read and summed.  The constants (us) are fitted
+// to every plan of six shapes (N, K from 576 x 7168 to 24576 x 1536) at 15 row
+// counts from 33 to 2048, weights cold; the estimate picks within 5% of the
+// fastest measured plan on all but a few, where it had been up to 1.9x off by
+// counting tiles alone: 193 x 18432 x 7168 64-row tiles in two rounds 77.1 us,
+// 256-row tiles split 3 ways in one 54.9; 512 x 1536 x 7168 256-row tiles split 8
+// ways 33.7, 64-row tiles split 5 ways 22.5; 768 x 4096 x 4096 41.1 / 27.1.
+static float dense_a8_time(const DenseA8Plan& p, int64_t m, int64_t n, int64_t k) {
+  const int64_t rows = std::min<int64_t>(m, p.tr), nch = k / 512;
+  const float steps = 4.f * (float)((nch + p.splits - 1) / p.splits);
+  const float rounds = (float)(((int64_t)p.n_row * p.n_col * p.splits + 255) / 256);
+  // a step's cost by the rows multiplied (256-row tiles: waves own 64-row quarters)
+  const float t = rows <= 64 ? 4.f + rounds * (1.f + (0.55f + 0.15f * (float)m / (64.f * p.n_row)) * steps)
+                             : 5.f + rounds * (5.f + (rows <= 128 ? 1.02f : rows <= 192 ? 1.1f : 1.54f) * steps);
+  return p.splits == 1 ? t : t + 2.f + 8.f * (float)p.splits * (float)m * (float)n / 5.5e6f;
 }
 static DenseA8Plan dense_a8_plan(int64_t m, int64_t n, int64_t k) {
-  if (m > 256) return dense_a8_plan_tr(m, n, k, 256);
-  // up to 256 rows: 64-row tiles, unless they leave over a third of the CUs idle
-  // and one 256-row tile per column (split further) fills more of them
-  // (128 x 18432 x 7168: 144 workgroups at 44.4 us, 216 at 40.5 us)
-  const DenseA8Plan p64 = dense_a8_plan_tr(m, n, k, 64), p256 = dense_a8_plan_tr(m, n, k, 256);
-  const int w64 = p64.n_row * p64.n_col * p64.splits, w256 = p256.n_row * p256.n_col * p256.splits;
-  return (w64 < 160 && w256 > w64 && w256 <= 256) ? p256 : p64;
+  DenseA8Plan best{};
+  float best_t = 0.f;
+  for (int tr = m <= 2048 ? 64 : 256; tr <= 256; tr += 192) {  // (64-row tiles measured up to 2048 rows)
+    DenseA8Plan p;
+    p.tr = tr;
+    p.n_row = (int)((m + tr - 1) / tr);
+    p.n_col = (int)((n + 255) / 256);
+    p.row_fastest = tr == 64 ? 1 : 0;
+    for (p.splits = 1; p.splits <= (int)std::min<int64_t>(8, k / 512); ++p.splits) {
+      const float t = dense_a8_time(p, m, n, k);
+      if (best_t == 0.f || t < best_t) best = p, best_t = t;
+    }
+  }
+  return best;
 }
 
 // the staged dense kernel runs when K is whole 512-K chunks and the rows are

@@ -518,6 +518,26 @@ def test_mxt16_linear_a8_prefill_vs_oracle(dev, m, n, k):
     assert_close(y.float().cpu().numpy(), L.mx_linear_a8(x, p, s), what=f"a8 prefill {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("m,n,k,split", [
+    (257, 576, 3584, 7), (300, 1536, 2048, 4), (513, 528, 1024, 1), (321, 9232, 512, 1), (193, 18432, 1024, 1),
+    (2048, 272, 1024, 1), (2049, 272, 1024, 2), (140, 12304, 2048, 1)])
+def test_mxt16_linear_a8_estimated_plans(dev, m, n, k, split):
+    """Plans the time estimate picks: 64-row tiles above 256 rows, unsplit and split (the last tile of 1 and
+    of 64 rows), one round and two, N tails, and the 2048-row limit of 64-row tiles."""
+    from mosaic_amd import _lib
+    ops = _ops()
+    rng = np.random.default_rng(m + n + k + 11)
+    p, s = _quant_weights(rng, n, k)
+    x = C.round_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    ws = _lib.lib().mosaic_mxt16_linear_a8_workspace_bytes(m, n, k)
+    assert ws == (4 * m * n * split if split > 1 else 0)
+    y = ops.mxt16_linear_a8(T(x).to(torch.bfloat16), ops.mxt16_prepack(T(p), T(s)))
+    rows = np.unique(np.r_[0, 1, 62:66, m // 2, m - 2, m - 1, rng.integers(0, m, 40)])
+    rows = rows[rows < m]
+    assert_close(y.float().cpu().numpy()[rows], L.mx_linear_a8(x[rows], p, s), what=f"a8 plan {m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("m,n,k", [(128, 1024, 4096), (4096, 576, 2048)])
 def test_mxt16_linear_a8_split_plan_matches_unsplit(dev, m, n, k):
     """A split-K plan without its workspace runs unsplit (mosaic_mxt16_linear_a8);
