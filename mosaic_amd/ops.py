@@ -20,20 +20,24 @@ ACT_MODES = {"pow2": 0, "amax": 1, "hf": 2, "legacy": 3}
 RECIPES = {"ceil": 0, "floor": 1}
 
 
+# The helpers below run several times in every call; at decode sizes a call's
+# GPU work is a few microseconds, so they avoid building Stream and device
+# objects, ctypes wrappers and no-op views (a one-token linear: 9.1 -> 6.3 us a
+# call among others).
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _cuda(t: torch.Tensor, name: str) -> torch.Tensor:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor (mosaic_amd has no CPU path), got {t.device}")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _on_device(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -41,13 +45,15 @@ def _on_device(t: torch.Tensor, name: str) -> torch.Tensor:
     operands that are read through their strides)."""
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor (mosaic_amd has no CPU path), got {t.device}")
     return t
 
 
 def _u8(t: torch.Tensor, name: str) -> torch.Tensor:
     t = _cuda(t, name)
+    if t.dtype == torch.uint8:
+        return t
     if t.dtype in (torch.uint8, torch.int8, torch.float8_e8m0fnu, torch.float8_e4m3fn):
         return t.view(torch.uint8)
     if hasattr(torch, "float4_e2m1fn_x2") and t.dtype == torch.float4_e2m1fn_x2:
