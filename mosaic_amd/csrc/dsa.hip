@@ -1631,6 +1631,273 @@ __global__ void __launch_bounds__(256) mla_decode_split_kernel(
   }
 }
 
+// A split of at most 128 selected tokens of one row and 64 heads over an FP8
+// cache, all tokens at once: decode calls of a few rows are bound by the chain
+// of latencies of a split (ids, gather, conversion, scores, softmax, values),
+// which the block loop above pays once per 32 tokens.  Here each step runs once
+// over the whole split, on eight waves (two a SIMD, so that one's LDS reads
+// overlap the other's products).
+//
+//   * every thread loads its tokens' ids, then 8 16-byte pieces of latent rows
+//     with their scales and 2 of rope rows, straight to registers, and writes
+//     them to LDS as bf16 (rounded as act_quant_sim stores them; zeros for masked
+//     tokens);
+//   * wave w scores tokens 32 (w / 2) .. + 31 against heads 32 (w % 2) .. + 31
+//     (S^T = K Q^T: q in registers, each K fragment used for two head tiles); the
+//     heads' maxima over the four token quarters meet in LDS, then the
+//     probabilities go to LDS over the rope rows, which are no longer needed;
+//   * wave w multiplies all heads into columns 64 w .. + 63, V read out of the
+//     latent rows with transposing reads.
+// Partials are laid out as the block kernel's.  q goes through LDS first (its
+// fragments straight from memory cost 36 scattered loads a wave, 8 us of the
+// chain).  Measured: 8 rows x 128 heads x 2048 picks 27.9 us on the block kernel,
+// ~17 here; what is left is the chain itself (~24,000 cycles: ids and q 9,000,
+// conversion 4,000, scores 3,400, softmax 2,300, values 2,700, stores 1,800).
+constexpr int kMdTokens = 128;
+constexpr int kMdRow = kMlaDl + 8;   // bf16 per latent row in LDS
+constexpr int kMdRope = 64 + 8;      // bf16 per rope row
+constexpr int kMdPs = kMdTokens + 8; // bf16 per row of P
+static_assert(64 * kMdPs <= kMdTokens * kMdRope, "P overlays the rope rows");
+constexpr int kMdQCopies = 64 * (kMlaDl + 64) * 2 / 1024 / 8;  // 1 KB copies of q a wave
+static_assert(64 * (kMlaDl + 64) <= kMdTokens * kMdRow, "q is staged where the latent rows go");
+
+__global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* __restrict__ q, const MlaKv kv,
+                                                               const int32_t* __restrict__ idx,
+                                                               uint16_t* __restrict__ part_o,
+                                                               float* __restrict__ part_ml, int topk, float scale) {
+  constexpr int DQK = kMlaDl + 64, NS = DQK / 32, NSL = kMlaDl / 32;
+  __shared__ __attribute__((aligned(16))) uint16_t Kt[kMdTokens * kMdRow];
+  __shared__ __attribute__((aligned(16))) uint16_t Rp[kMdTokens * kMdRope];
+  __shared__ float Mx[4][64], Lx[4][64];
+  __shared__ int Live[kMdTokens];
+  const int H = 64 * gridDim.z;
+  const int split = blockIdx.x, b = blockIdx.y, S = gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, qd = lane >> 4;
+  const int64_t n = kv.n, kvb = (int64_t)(b / kv.rows_per_kv) * n;
+  const int t0 = split * kMdTokens, nt = min(kMdTokens, topk - t0);  // tokens of this split (> 0)
+  const int nblk = (nt + 31) / 32;
+  const int nsc = kMlaDl >> kv.sb_shift;
+  // the group's q rows (73,728 contiguous bytes) into LDS, each row's 16-byte
+  // chunks XOR-swizzled by (row / 2) % 8 within eights, so that the 16 rows of a
+  // fragment read fall in distinct banks
+  const int hh = wv & 1, tb = wv >> 1;
+  {
+    const uint16_t* qg = q + ((int64_t)b * H + 64 * blockIdx.z) * DQK;
+#pragma unroll
+    for (int i = 0; i < kMdQCopies; ++i) {
+      const int u = 64 * (kMdQCopies * wv + i) + lane, r = u / (DQK / 8), p = u - r * (DQK / 8);
+      mla_copy16(qg + r * DQK + 8 * (p ^ ((r >> 1) & 7)), mla_lds_addr(&Kt[512 * (kMdQCopies * wv + i)]));
+    }
+  }
+  // Wave wv gathers tokens 16 i + 2 wv + {0, 1}: latent piece i is token 2 wv +
+  // lane / 32 of the i-th 16, bytes 16 (lane % 32); rope piece j covers eight of
+  // the tokens, 8 values at 8 (lane % 8).  The ids are wave-uniform, so they come
+  // by scalar loads, which do not wait for q's copies.
+  const int32_t* ids = idx + (int64_t)b * topk + t0;
+  const int lp = lane & 31, rp = lane & 7, lt = 2 * wv + (lane >> 5);
+  int id2[8][2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) id2[i][u] = ids[min(16 * i + 2 * wv + u, nt - 1)];
+  __builtin_amdgcn_sched_barrier(0);  // all loads first: one wait instead of sixteen
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)  // (a negative id stays negative)
+      id2[i][u] = 16 * i + 2 * wv + u < nt && (int64_t)id2[i][u] < n ? id2[i][u] : -1;
+  int lid[8], rid[2], rt[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) lid[i] = lane < 32 ? id2[i][0] : id2[i][1];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    rid[j] = id2[4 * j][0];
+#pragma unroll
+    for (int g = 1; g < 8; ++g) rid[j] = (lane >> 3) == g ? id2[4 * j + (g >> 1)][g & 1] : rid[j];
+    rt[j] = 16 * (4 * j + (lane >> 4)) + 2 * wv + ((lane >> 3) & 1);
+  }
+  // masked tokens read row 0 and are zeroed below (loads under a branch would be
+  // waited for at its end)
+  u32x4_t raw[8], rope[2];
+  float sc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int64_t r = kvb + max(lid[i], 0);
+    raw[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(kv.lat) + r * kMlaDl + 16 * lp);
+    sc[i] = kv.lat_s[r * nsc + ((16 * lp) >> kv.sb_shift)];
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    rope[i] = *reinterpret_cast<const u32x4_t*>(kv.rope + (kvb + max(rid[i], 0)) * 64 + 8 * rp);
+  }
+  // q has landed (the gather may still fly); it becomes the B operand of S^T:
+  // heads 32 hh + 16 t + c of the group
+  asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
+  bf16x8_t qf[2][NS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = 32 * hh + 16 * t + c;
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      qf[t][s] = *reinterpret_cast<const bf16x8_t*>(&Kt[r * DQK + 8 * ((4 * s + qd) ^ ((r >> 1) & 7))]);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // q's LDS may be overwritten
+  if (lp == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) Live[16 * i + lt] = lid[i] >= 0 ? 1 : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    uint32_t o[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // exact e4m3 -> fp32, fp32 product with the scale, one RNE rounding to bf16
+      f32x2_t a2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)raw[i][e], false);
+      f32x2_t b2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)raw[i][e], true);
+      a2[0] *= sc[i];
+      a2[1] *= sc[i];
+      b2[0] *= sc[i];
+      b2[1] *= sc[i];
+      o[2 * e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(a2, bf16x2_t));
+      o[2 * e + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(b2, bf16x2_t));
+    }
+    u32x4_t* dst = reinterpret_cast<u32x4_t*>(&Kt[(16 * i + lt) * kMdRow + 16 * lp]);
+    const bool ok = lid[i] >= 0;
+    dst[0] = ok ? u32x4_t{o[0], o[1], o[2], o[3]} : u32x4_t{0u, 0u, 0u, 0u};
+    dst[1] = ok ? u32x4_t{o[4], o[5], o[6], o[7]} : u32x4_t{0u, 0u, 0u, 0u};
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    *reinterpret_cast<u32x4_t*>(&Rp[rt[i] * kMdRope + 8 * rp]) = rid[i] >= 0 ? rope[i] : u32x4_t{0u, 0u, 0u, 0u};
+  }
+  __syncthreads();
+  // scores of this wave's 32 tokens (slot order, see mla_slot_token) x 32 heads
+  f32x4_t st[2][2];  // [head tile][slot tile]
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) st[t][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  bool live[2][4];
+  const bool scorer = tb < nblk;
+  if (scorer) {
+    int krow[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      krow[j] = 32 * tb + mla_slot_token(16 * j + c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) live[j][r] = Live[32 * tb + mla_slot_token(16 * j + 4 * qd + r)] != 0;
+    }
+    // K fragments in batches of KB steps, one batch ahead of the products
+    constexpr int KB = 3, NKB = NS / KB;
+    bf16x8_t kf[2][KB][2];
+    auto read_k = [&](int kb2, bf16x8_t (&dst)[KB][2]) {
+#pragma unroll
+      for (int ss = 0; ss < KB; ++ss)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int s = kb2 * KB + ss;
+          dst[ss][j] = *reinterpret_cast<const bf16x8_t*>(s < NSL ? &Kt[krow[j] * kMdRow + 32 * s + 8 * qd]
+                                                                  : &Rp[krow[j] * kMdRope + 32 * (s - NSL) + 8 * qd]);
+        }
+    };
+    read_k(0, kf[0]);
+#pragma unroll
+    for (int kb2 = 0; kb2 < NKB; ++kb2) {
+      if (kb2 + 1 < NKB) read_k(kb2 + 1, kf[(kb2 + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ss = 0; ss < KB; ++ss)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) st[t][j] = mfma_bf16(kf[kb2 & 1][ss][j], qf[t][kb2 * KB + ss], st[t][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    float bm = -INFINITY;
+    if (scorer) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          st[t][j][r] = live[j][r] ? st[t][j][r] * scale : -INFINITY;
+          bm = fmaxf(bm, st[t][j][r]);
+        }
+      bm = fmaxf(bm, __shfl_xor(bm, 16));
+      bm = fmaxf(bm, __shfl_xor(bm, 32));
+    }
+    if (qd == 0) Mx[tb][32 * hh + 16 * t + c] = bm;
+  }
+  __syncthreads();  // the maxima are in, and no wave reads the rope rows any more
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int hd = 32 * hh + 16 * t + c;
+    const float m = fmaxf(fmaxf(Mx[0][hd], Mx[1][hd]), fmaxf(Mx[2][hd], Mx[3][hd]));
+    float l = 0.f;
+    if (scorer) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          p[r] = m == -INFINITY ? 0.f : __expf(st[t][j][r] - m);
+          l += p[r];
+        }
+        *reinterpret_cast<uint2*>(&Rp[hd * kMdPs + 32 * tb + 16 * j + 4 * qd]) =
+            uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{p[0], p[1]}, bf16x2_t)),
+                  __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{p[2], p[3]}, bf16x2_t))};
+      }
+      l += __shfl_xor(l, 16);
+      l += __shfl_xor(l, 32);
+    }
+    if (qd == 0) Lx[tb][hd] = l;
+  }
+  __syncthreads();
+  // O = P V over this wave's 64 columns
+  f32x4_t o[4][4];
+#pragma unroll
+  for (int ht = 0; ht < 4; ++ht)
+#pragma unroll
+    for (int dl = 0; dl < 4; ++dl) o[ht][dl] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int vi = c >> 2, vj = c & 3;
+  for (int bk = 0; bk < nblk; ++bk) {
+    bf16x8_t pa[4], vv[4];
+#pragma unroll
+    for (int ht = 0; ht < 4; ++ht)
+      pa[ht] = *reinterpret_cast<const bf16x8_t*>(&Rp[(16 * ht + c) * kMdPs + 32 * bk + 8 * qd]);
+#pragma unroll
+    for (int dl = 0; dl < 4; ++dl) {
+      const uint16_t* vp = &Kt[(32 * bk + 8 * qd + 2 * vi) * kMdRow + 4 * vj + 64 * wv + 16 * dl];
+      const mla_v4s a = lds_read_tr16(vp), e = lds_read_tr16(vp + kMdRow);
+      vv[dl] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, e, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+#pragma unroll
+    for (int dl = 0; dl < 4; ++dl)
+#pragma unroll
+      for (int ht = 0; ht < 4; ++ht) o[ht][dl] = mfma_bf16(pa[ht], vv[dl], o[ht][dl]);
+  }
+  uint16_t* po = part_o + ((int64_t)b * S + split) * (H / 16) * (kMlaDt * 256);
+#pragma unroll
+  for (int ht = 0; ht < 4; ++ht)
+#pragma unroll
+    for (int dl = 0; dl < 4; ++dl) {
+      const f32x4_t v = o[ht][dl];
+      *reinterpret_cast<uint2*>(po + (((int64_t)(4 * blockIdx.z + ht) * kMlaDt + 4 * wv + dl) * 64 + lane) * 4) =
+          uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[0], v[1]}, bf16x2_t)),
+                __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[2], v[3]}, bf16x2_t))};
+    }
+  if (tid < 64) {
+    const float m = fmaxf(fmaxf(Mx[0][tid], Mx[1][tid]), fmaxf(Mx[2][tid], Mx[3][tid]));
+    const float l = (Lx[0][tid] + Lx[1][tid]) + (Lx[2][tid] + Lx[3][tid]);
+    float* pml = part_ml + (((int64_t)b * S + split) * H + 64 * blockIdx.z + tid) * 2;
+    *reinterpret_cast<f32x2_t*>(pml) = f32x2_t{m, l};
+  }
+}
+
 // Merge the splits of one (row, 16-head tile, 16-column tile) with the sink
 // term and normalize.  Each wave turns the split maxima/sums of four heads
 // into weights (lane = split); then wave w blends splits w, w + 4, ... of the
@@ -2305,8 +2572,20 @@ static int mla_head_tiles(int64_t b, int64_t h, int S) {
   while (ht > 1 && (h / 16) % (ht / 2) == 0 && (int64_t)S * b * (h / (16 * ht)) < 256) ht /= 2;
   return ht;
 }
+// Splits of the whole-split kernel (kMdTokens selected tokens each), 0 where the
+// block kernel runs: it takes groups of 64 heads, and from 24 to 1024 workgroups
+// (us, block kernel against whole splits, 128 heads unless said: 8 rows of 2048
+// picks 34.1 / 23.6, 3 rows 31.5 / 18.8, 12 rows 60.9 / 35.6, 3 rows of 512 22.3 /
+// 16.1; below, the block kernel spreads 16-head groups wider: 2 rows of 512 14.7 /
+// 15.4, 64 heads x 4 rows of 512 14.6 / 15.4; above, its fewer partials win: 32
+// rows of 4096 128 / 139).
+static int mla_chunks(int64_t b, int64_t h, int64_t topk) {
+  const int64_t chunks = (topk + kMdTokens - 1) / kMdTokens;
+  const int64_t wgs = b * (h / 64) * chunks;
+  return h % 64 == 0 && chunks <= 32 && b <= 32 && wgs >= 24 && wgs <= 1024 ? (int)chunks : 0;
+}
 static size_t mla_ws(int64_t b, int64_t h, int64_t topk, char* base, MlaWs* w) {
-  const int64_t S = mla_splits(b, topk);
+  const int64_t S = std::max(mla_splits(b, topk), mla_chunks(b, h, topk));
   const size_t ob = align256((size_t)b * S * h * kMlaDl * 2);
   const size_t mb = align256((size_t)b * S * h * 2 * 4);
   if (w) {
@@ -2436,21 +2715,29 @@ static int launch_mla(const uint16_t* q, const MlaKv& kv, const float* sink, con
                       int64_t rows, int64_t h, int64_t topk, float softmax_scale, void* workspace, hipStream_t st) {
   MlaWs ws;
   mla_ws(rows, h, topk, (char*)workspace, &ws);
-  const int S = mla_splits(rows, topk);
-  const int blocks = (int)((topk + kMlaBT - 1) / kMlaBT);
-  const int chunk = ((blocks + S - 1) / S) * kMlaBT;
-  const int ht = mla_head_tiles(rows, h, S);
-  dim3 grid((unsigned)S, (unsigned)rows, (unsigned)(h / (16 * ht)));
-  switch (ht) {
+  int S = mla_splits(rows, topk);
+  const int chunks = FP8 && kv.n > 0 ? mla_chunks(rows, h, topk) : 0;
+  if (chunks > 0) {
+    S = chunks;
+    MOSAIC_LAUNCH(mla_decode_chunk_kernel, dim3((unsigned)S, (unsigned)rows, (unsigned)(h / 64)), dim3(512), 0, st, q,
+                  kv, idx, ws.part_o, ws.part_ml, (int)topk, softmax_scale);
+    MOSAIC_LAUNCH_CHECK("mla_decode_chunk");
+  } else {
+    const int blocks = (int)((topk + kMlaBT - 1) / kMlaBT);
+    const int chunk = ((blocks + S - 1) / S) * kMlaBT;
+    const int ht = mla_head_tiles(rows, h, S);
+    dim3 grid((unsigned)S, (unsigned)rows, (unsigned)(h / (16 * ht)));
+    switch (ht) {
 #define MLA_CASE(HTV)                                                                                                  \
   case HTV:                                                                                                            \
     MOSAIC_LAUNCH((mla_decode_split_kernel<HTV, FP8, DR>), grid, dim3(256), 0, st, q, kv, idx, ws.part_o,       \
                        ws.part_ml, (int)topk, softmax_scale, chunk);                                                   \
     break;
-    MLA_CASE(1) MLA_CASE(2) MLA_CASE(3) MLA_CASE(4)
+      MLA_CASE(1) MLA_CASE(2) MLA_CASE(3) MLA_CASE(4)
 #undef MLA_CASE
+    }
+    MOSAIC_LAUNCH_CHECK("mla_decode_split");
   }
-  MOSAIC_LAUNCH_CHECK("mla_decode_split");
   if (rows * (h / 16) * (kMlaDt / kMlaCombineTiles) >= 256)
     MOSAIC_LAUNCH(mla_combine_tiles_kernel,
                   dim3((unsigned)(kMlaDt / kMlaCombineTiles), (unsigned)(h / 16), (unsigned)rows), dim3(256), 0, st,

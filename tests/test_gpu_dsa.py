@@ -235,6 +235,25 @@ def test_mla_fp8_vs_oracle(dev, b, h, n, t, sb, sink, masked):
     _close(out.float().cpu().numpy(), D.mla_sparse_decode(q, lat, ls, rope, snk, idx, scale, sb))
 
 
+@pytest.mark.parametrize("b,h,n,t,sb,masked", [
+    (24, 64, 50, 1, 64, 0.0), (24, 64, 300, 31, 16, 0.3), (12, 128, 500, 129, 512, 0.0), (6, 256, 400, 128, 128, 0.6),
+    (8, 128, 700, 300, 64, 0.2), (2, 192, 4200, 4096, 32, 0.0), (32, 64, 900, 257, 64, 0.9)])
+def test_mla_fp8_whole_splits_vs_oracle(dev, b, h, n, t, sb, masked):
+    """The whole-split kernel: splits of 1, 31, 128 and few tokens (idle scoring waves), several head groups,
+    every scale-block size class, masked picks, picks past the cache, a row without a valid pick and a
+    split without one."""
+    from mosaic_amd import ops
+    rng = np.random.default_rng(b * 100 + t)
+    q, lat, ls, rope, idx = _mla(rng, b, h, n, t, sb, masked)
+    idx[1] = -1
+    idx[0, 128:256] = n + 3
+    snk = rng.standard_normal(h).astype(np.float32)
+    qd, latd, lsd, rd, idxd = _t(dev, q, lat, ls, rope, idx)
+    out = ops.mla_sparse_decode(qd.to(torch.bfloat16), latd, lsd, rd.to(torch.bfloat16), idxd, 0.06,
+                                torch.from_numpy(snk).to(dev))
+    _close(out.float().cpu().numpy(), D.mla_sparse_decode(q, lat, ls, rope, snk, idx, 0.06, sb))
+
+
 def test_mla_wide_score_range(dev):
     """Scores rising by over a hundred nats along the token order (the rope part
     grows 300-fold): every head's running maximum moves past the lazy margin
