@@ -295,9 +295,9 @@ static void launch_fp8_skinny(const uint8_t* a, const float* as, const uint8_t* 
                      (int)k, out_f32);
 }
 
-// Tiled kernel (M >= 96, MFMA-bound at large M): a workgroup of BM/32 waves
+// Tiled kernel (M >= 96, MFMA-bound at large M): a workgroup of BM/16 waves
 // owns a BM x 128 block of C (its 128 columns share one b_s row); each wave
-// owns a 64x64 quarter (4x4 MFMA tiles).  Each 128-K block's A and B tiles and
+// owns a 64x32 part (4x2 MFMA tiles).  Each 128-K block's A and B tiles and
 // its scales (BM a_s values, one b_s) go global -> LDS directly
 // (global_load_lds, 16 bytes a lane into 1 KB runs, 4 bytes a lane for the
 // scales) through a ring of three stages, two blocks ahead of the MFMAs.  All
@@ -313,7 +313,18 @@ static void launch_fp8_skinny(const uint8_t* a, const float* as, const uint8_t* 
 // schedule: transposed MFMA roles (one a_s per lane and tile, 4 consecutive C
 // columns per lane), the next A fragment read during the MFMAs, each tile's
 // rescale issued after the next tile's MFMAs.
-constexpr int kTileN = 128, kStages = 3;
+// Each wave owns 64 x 32 of the tile, so a 128-row workgroup has two waves a SIMD
+// and a 256-row one four: with 64 x 64 a wave (half as many) each wave's chain of
+// LDS reads, MFMAs and rescales stood alone on its SIMD between two barriers
+// (us, 64 x 64 against 64 x 32: 65 x 18432 x 7168 54.8 / 46.8, 1024 x 4096 x 4096
+// 35.4 / 30.9, 2048 x 1536 x 7168 54.3 / 46.5; 256-row tiles 256 x 18432 x 7168
+// 81.2 / 74.5, 1024 x 7168 x 16384 172.8 / 164.7).
+// The copies of block i + 2 go out during block i, at row tile ISSUE: the last one
+// for a single 128-row tile, whose workgroups all stream their own weights (at the
+// first one their issue holds up the MFMAs while the ring is full of loads), else
+// the first (us, first / last: 128 x 18432 x 7168 54.9 / 51.8, 128 x 7168 x 16384
+// 48.4 / 46.0; 200 x 18432 x 7168 74.1 / 77.7, 768 x 4096 x 4096 27.5 / 31.0).
+constexpr int kTileN = 128, kTileWN = 32, kStages = 3;
 
 __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int T = tiles_m * tiles_n;
@@ -353,8 +364,9 @@ __device__ __forceinline__ void fp8_copy4(const void* g, uint32_t lds) {
 
 template <int BM>
 struct Fp8Tile {
-  static constexpr int NT = BM * 2;                   // threads
-  static constexpr int NW = NT / 64;                  // waves
+  static constexpr int NWN = kTileN / kTileWN;        // waves across the columns
+  static constexpr int NW = BM / 64 * NWN;            // waves
+  static constexpr int NT = NW * 64;                  // threads
   static constexpr int AB = (BM + kTileN) * 128;      // A and B bytes of a stage
   static constexpr int SA = AB;                       // a_s: BM floats
   static constexpr int SB = SA + BM * 4;              // b_s: 64 copies of one float
@@ -369,19 +381,20 @@ struct Fp8Tile {
 // Split-K (blockIdx.y = K slice of kps blocks): with `part` the slice writes its
 // fp32 partial tile to part[slice][M][N] (fp8_splitk_reduce_kernel sums the
 // slices in order); without it the tile goes to C.
-template <int BM>
-__global__ void __launch_bounds__(BM * 2, 1) fp8_gemm_tiled_kernel(
+template <int BM, int ISSUE>
+__global__ void __launch_bounds__(BM * kTileN / kTileWN, 1) fp8_gemm_tiled_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ B,
     const float* __restrict__ Bs, void* __restrict__ C, int M, int N, int K, int out_f32, int kps,
     float* __restrict__ part) {
   using TT = Fp8Tile<BM>;
+  constexpr int CT = kTileWN / 16;  // column tiles a wave
   __shared__ __attribute__((aligned(16))) uint8_t lds[kStages][TT::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int c = lane & 15, q = lane >> 4;
   int tm, tn;
   tile_coords(blockIdx.x, (M + BM - 1) / BM, (N + kTileN - 1) / kTileN, tm, tn);
   const int m0 = tm * BM, n0 = tn * kTileN;
-  const int wm = (wv >> 1) * 64, wn = (wv & 1) * 64;
+  const int wm = wv / TT::NWN * 64, wn = wv % TT::NWN * kTileWN;
   const int nkb = K / 128;
   // this lane's source row and 16-byte chunk for each of the wave's A/B runs
   const uint8_t* gsrc[TT::RUNS];
@@ -412,14 +425,14 @@ __global__ void __launch_bounds__(BM * 2, 1) fp8_gemm_tiled_kernel(
     for (int ii = 0; ii < TT::RUNS; ++ii) fp8_copy16(gsrc[ii] + (int64_t)kb * 128, base + ldsoff[ii]);
     fp8_copy4(ssrc + kb, base + sdst);
   };
-  f32x4_t acc[4][4];
+  f32x4_t acc[4][CT];
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  f32x4_t dp[4];  // product of the previous tile, rescaled one tile later
+    for (int nt = 0; nt < CT; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t dp[CT];  // product of the previous tile, rescaled one tile later
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) dp[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int nt = 0; nt < CT; ++nt) dp[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float sp = 0.f;
   const int kb0 = (int)blockIdx.y * kps, cnt = min(nkb, kb0 + kps) - kb0;
   // a slice past K (never launched) copies nothing and writes zero partials
@@ -431,35 +444,39 @@ __global__ void __launch_bounds__(BM * 2, 1) fp8_gemm_tiled_kernel(
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::"n"(TT::OPS) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (i + 2 < cnt) issue((i + 2) % kStages, kb0 + i + 2);
     const uint8_t* stg = lds[i % kStages];
     const uint8_t* ta = stg;
     const uint8_t* tb = stg + BM * 128;
     const float sb = *reinterpret_cast<const float*>(stg + TT::SB);
-    i32x8_t bop[4];
+    i32x8_t bop[CT];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) bop[nt] = lds_fp8_operand(tb, wn + 16 * nt + c, q);
+    for (int nt = 0; nt < CT; ++nt) bop[nt] = lds_fp8_operand(tb, wn + 16 * nt + c, q);
     i32x8_t aop[2];
     aop[0] = lds_fp8_operand(ta, wm + c, q);
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       if (mt + 1 < 4) aop[(mt + 1) & 1] = lds_fp8_operand(ta, wm + 16 * (mt + 1) + c, q);
       // transposed roles: rows are B rows (n), columns A rows (m = wm + 16 mt + c)
-      f32x4_t d[4];
+      f32x4_t d[CT];
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) d[nt] = mfma_fp8_block(bop[nt], aop[mt & 1]);
+      for (int nt = 0; nt < CT; ++nt) d[nt] = mfma_fp8_block(bop[nt], aop[mt & 1]);
+      if (mt == ISSUE) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < cnt) issue((i + 2) % kStages, kb0 + i + 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       const int pm = mt == 0 ? 3 : mt - 1;  // the previous tile (tile 3 of the previous block at mt == 0)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+      for (int nt = 0; nt < CT; ++nt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[pm][nt][r] = __builtin_fmaf(dp[nt][r], sp, acc[pm][nt][r]);
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) dp[nt] = d[nt];
+      for (int nt = 0; nt < CT; ++nt) dp[nt] = d[nt];
       sp = *reinterpret_cast<const float*>(stg + TT::SA + 4 * (wm + 16 * mt + c)) * sb;
     }
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < CT; ++nt)
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[3][nt][r] = __builtin_fmaf(dp[nt][r], sp, acc[3][nt][r]);
   // lane (c, q) of tile (mt, nt) holds C[m0 + wm + 16 mt + c][n .. n + 3], n = n0 + wn + 16 nt + 4 q
@@ -470,7 +487,7 @@ __global__ void __launch_bounds__(BM * 2, 1) fp8_gemm_tiled_kernel(
     const int m = m0 + wm + 16 * mt + c;
     if (m >= M) continue;
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
+    for (int nt = 0; nt < CT; ++nt) {
       const int n = n0 + wn + 16 * nt + 4 * q;
       const f32x4_t v = acc[mt][nt];
       if (part || out_f32) {
@@ -498,21 +515,50 @@ __global__ void __launch_bounds__(BM * 2, 1) fp8_gemm_tiled_kernel(
   }
 }
 
-// C = sum over the S slices of part, in slice order; 4 elements per thread
+// C = sum over the S (at most 8) slices of part, in slice order; 4 elements per
+// thread.  Where rows of 4 stay aligned (VEC) every slice's 16 bytes are loaded
+// before the sum.
+template <bool VEC>
 __global__ void __launch_bounds__(256) fp8_splitk_reduce_kernel(const float* __restrict__ part, int S, int64_t mn,
                                                                 void* __restrict__ C, int out_f32) {
   const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if constexpr (VEC) {
+    if (i0 >= mn) return;
+    f32x4_t p[8];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t i = i0 + j;
-    if (i >= mn) break;
-    float v = part[i];
-    for (int sl = 1; sl < S; ++sl) v += part[(int64_t)sl * mn + i];
+    for (int sl = 0; sl < 8; ++sl)
+      if (sl < S) p[sl] = *reinterpret_cast<const f32x4_t*>(part + (int64_t)sl * mn + i0);
+    f32x4_t v = p[0];
+#pragma unroll
+    for (int sl = 1; sl < 8; ++sl)
+      if (sl < S) v += p[sl];
     if (out_f32)
-      reinterpret_cast<float*>(C)[i] = v;
+      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(C) + i0) = v;
     else
-      reinterpret_cast<uint16_t*>(C)[i] = f32_bf16(v);
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(C) + i0) =
+          make_uint2((uint32_t)f32_bf16(v[0]) | ((uint32_t)f32_bf16(v[1]) << 16),
+                     (uint32_t)f32_bf16(v[2]) | ((uint32_t)f32_bf16(v[3]) << 16));
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t i = i0 + j;
+      if (i >= mn) break;
+      float v = part[i];
+      for (int sl = 1; sl < S; ++sl) v += part[(int64_t)sl * mn + i];
+      if (out_f32)
+        reinterpret_cast<float*>(C)[i] = v;
+      else
+        reinterpret_cast<uint16_t*>(C)[i] = f32_bf16(v);
+    }
   }
+}
+
+static void launch_fp8_reduce(const float* part, int S, int64_t mn, void* c, int out_f32, hipStream_t st) {
+  const dim3 grid((unsigned)((mn + 1023) / 1024));
+  if (mn % 4 == 0 && S <= 8 && ((uintptr_t)part | (uintptr_t)c) % 16 == 0)
+    MOSAIC_LAUNCH(fp8_splitk_reduce_kernel<true>, grid, dim3(256), 0, st, part, S, mn, c, out_f32);
+  else
+    MOSAIC_LAUNCH(fp8_splitk_reduce_kernel<false>, grid, dim3(256), 0, st, part, S, mn, c, out_f32);
 }
 
 template <int BM>
@@ -524,13 +570,15 @@ static void launch_fp8_tiled(const uint8_t* a, const float* as, const uint8_t* b
   // slices of kps blocks: only the non-empty ones are launched (K = 33 blocks
   // in 8 slices of 5 would leave slice 7 starting past K)
   S = (nkb + kps - 1) / kps;
-  MOSAIC_LAUNCH((fp8_gemm_tiled_kernel<BM>), dim3((unsigned)tiles, (unsigned)S), dim3(BM * 2), 0, st, a, as, b,
-                     bs, c, (int)m, (int)n, (int)k, out_f32, kps, S > 1 ? part : nullptr);
-  if (S > 1) {
-    const int64_t mn = m * n;
-    MOSAIC_LAUNCH(fp8_splitk_reduce_kernel, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, st, part, S, mn,
-                       c, out_f32);
-  }
+  const dim3 grid((unsigned)tiles, (unsigned)S), block(Fp8Tile<BM>::NT);
+  float* p = S > 1 ? part : nullptr;
+  if (BM == 128 && m <= BM)
+    MOSAIC_LAUNCH((fp8_gemm_tiled_kernel<128, 3>), grid, block, 0, st, a, as, b, bs, c, (int)m, (int)n, (int)k,
+                  out_f32, kps, p);
+  else
+    MOSAIC_LAUNCH((fp8_gemm_tiled_kernel<BM, 0>), grid, block, 0, st, a, as, b, bs, c, (int)m, (int)n, (int)k,
+                  out_f32, kps, p);
+  if (S > 1) launch_fp8_reduce(part, S, m * n, c, out_f32, st);
 }
 
 // Mid-size kernel (16 < M <= 64): the decode ring's weight stream with G
@@ -760,11 +808,7 @@ static void launch_fp8_mid(const uint8_t* a, const float* as, const uint8_t* b, 
   }
 #undef FP8_MID_W
 #undef FP8_MID
-  if (S > 1) {
-    const int64_t mn = m * n;
-    MOSAIC_LAUNCH(fp8_splitk_reduce_kernel, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, st, part, S, mn, c,
-                  out_f32);
-  }
+  if (S > 1) launch_fp8_reduce(part, S, m * n, c, out_f32, st);
 }
 
 // Large tiled kernel (enough 256 x 256 tiles to fill the chip): a workgroup
@@ -1037,24 +1081,45 @@ extern "C" int mosaic_fp8_block_dequant(const uint8_t* w, const float* s, uint16
 struct Fp8Plan {
   int kind, S;
 };
+// Estimated time (us) of a tiled plan: rounds of at most 256 workgroups (each
+// kernel's LDS leaves one a CU) of a fixed part and K blocks, the blocks dearer
+// where more distinct weight streams run at once, plus the split's partials
+// written, read and summed.  The constants are fitted to every plan of six shapes
+// (576 x 7168 to 24576 x 1536 and 7168 x 16384) at 12 row counts from 65 to 2048,
+// weights cold; the pick is within 10% of the fastest measured plan on all of
+// them but 96 x 4096 x 4096, and 1.13x faster on average than the rule by tile
+// counts before (us, before / now: 300 x 18432 x 7168 143.8 / 92.1, 512 rows 159.5
+// / 109.6, 2048 x 7168 x 16384 342 / 227, 256 x 576 x 7168 21.1 / 16.8).
+static float fp8_tiled_time(int kind, int S, int64_t m, int64_t n, int64_t k) {
+  const int64_t bm = kind == 1 ? 128 : 256, bn = kind == 3 ? 256 : 128, nkb = k / 128;
+  const int64_t steps = (nkb + S - 1) / S, slices = (nkb + steps - 1) / steps, n_row = (m + bm - 1) / bm;
+  const int64_t wgs = n_row * ((n + bn - 1) / bn) * slices;
+  const float streams = (float)std::min<int64_t>(256, wgs) / (256.f * (float)n_row);
+  const float fixed = kind == 1 ? 4.f : kind == 2 ? 5.f : 6.f, round = kind == 3 ? 4.f : 1.f;
+  const float step = kind == 1   ? 0.68f + 0.30f * streams
+                     : kind == 2 ? 1.20f + 0.25f * streams
+                                 : 1.65f + 0.35f * streams;
+  const float t = fixed + (float)((wgs + 255) / 256) * (round + step * (float)steps);
+  return slices == 1 ? t : t + 2.f + 8.f * (float)slices * (float)m * (float)n / 5.5e6f;
+}
 static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k) {
   const int64_t nkb = k / 128;
-  auto split = [&](int64_t tiles) {
-    int64_t s = std::min<int64_t>(8, std::min<int64_t>(256 / std::max<int64_t>(tiles, 1), nkb / 4));
-    return tiles * 2 <= 256 && s >= 2 ? (int)s : 1;
-  };
-  if (m >= 256) {
-    const int64_t big_tiles = ((m + 255) / 256) * ((n + 255) / 256);
-    // the big kernel addresses A and B with 32-bit offsets
-    if (big_tiles >= 256 && m * k < (1ll << 32) && n * k < (1ll << 32)) return {3, 1};
-    return {2, split(((m + 255) / 256) * ((n + 127) / 128))};
-  }
-  // 65..95 rows: the tiled kernel for weights of 8 MB and more (18432 x 7168:
-  // 180 -> 55 us), the skinny kernel below (576 x 7168: 11.7 against 16.9 us)
+  // Tiled kernels from 96 rows; at 65..95 rows for weights of 8 MB and more (18432
+  // x 7168: 180 -> 46 us; 576 x 7168: the skinny kernel's 11.7 against 14.5 us).
+  // 256-row tiles pay from 129 rows.
   if (m >= 96 || (m > 64 && n * k >= (8ll << 20))) {
+    Fp8Plan best{0, 1};
+    float best_t = 0.f;
+    for (int kind = 1; kind <= (m > 128 ? 3 : 1); ++kind) {
+      // the 256 x 256 kernel addresses A and B with 32-bit offsets and does not split K
+      if (kind == 3 && (m * k >= (1ll << 32) || n * k >= (1ll << 32))) continue;
+      for (int S = 1; S <= (kind == 3 ? 1 : 8) && (S == 1 || nkb / S >= 4); ++S) {
+        const float t = fp8_tiled_time(kind, S, m, n, k);
+        if (best_t == 0.f || t < best_t) best = Fp8Plan{kind, S}, best_t = t;
+      }
+    }
     const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    const int s = split(tiles);
-    if (tiles * s >= 32) return {1, s};
+    if (m >= 256 || best.kind != 1 || tiles * best.S >= 32) return best;
   }
   // decode shapes: the ring kernel for wide N, and for narrower N when K is deep
   // enough for its 8-wave split to leave each wave >= 4 blocks (M = 1 / 16,

@@ -67,6 +67,27 @@ def test_fp8_block_gemm_vs_oracle(dev, m, n, k, out):
         assert viol.max() <= 0, f"f32 reassociation bound exceeded by {viol.max()} (max scaled err {err.max()})"
 
 
+@pytest.mark.parametrize("out", ["bf16", "f32"])
+@pytest.mark.parametrize("m,n,k", [
+    # 256-row tiles from 129 rows (ragged M and N, two rounds of workgroups, one and two K blocks a stage ring)
+    (129, 33000, 128), (200, 24592, 256), (255, 20000, 1024), (500, 9000, 640),
+    # 128-row tiles above 256 rows, unsplit and split 8, 7 and 2 ways (N % 4 != 0: the scalar reduce)
+    (257, 576, 4096), (300, 1536, 3584), (321, 2050, 1024), (770, 1030, 1024), (300, 18448, 512),
+    # the 256 x 256 kernel on fewer than 256 tiles, ragged
+    (300, 24590, 1024)])
+def test_fp8_block_gemm_estimated_plans(dev, m, n, k, out):
+    """Plans the time estimate picks that the tile counts did not: sampled rows against the oracle."""
+    from mosaic_amd import ops
+    rng = np.random.default_rng(m + n + k)
+    aq, a_s, bq, bs = _case(rng, m, n, k)
+    T = lambda v: torch.from_numpy(np.ascontiguousarray(v)).to(dev)
+    c = ops.fp8_block_gemm(T(aq), T(a_s), T(bq), T(bs), out_dtype=torch.bfloat16 if out == "bf16" else torch.float32)
+    rows = np.unique(np.r_[0, 1, 63, 64, 127, 128, m // 2, m - 2, m - 1, rng.integers(0, m, 24)])
+    ref = L.fp8_block_gemm(aq[rows], a_s[rows], bq, bs, out_bf16=(out == "bf16"))
+    err = np.abs(c.float().cpu().numpy()[rows] - ref) / np.maximum(1.0, np.abs(ref))
+    assert err.max() <= 2e-2, f"max scaled err {err.max()}"
+
+
 @pytest.mark.parametrize("m,n,k,e8m0", [(1, 1536, 7168, False), (1, 18432, 7168, True), (16, 576, 7168, False),
                                         (37, 200, 1024, True), (80, 4096, 512, False), (3, 24576, 1536, True),
                                         (5, 16, 128, False),
