@@ -42,6 +42,7 @@
 //   e4m3 * scale -> bf16, rope bf16], v_t = latent.  Online softmax over 32-token
 //   blocks in each of several token splits, then a combine over splits.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "../../include/mosaic_amd.h"
@@ -1631,6 +1632,28 @@ __global__ void __launch_bounds__(256) mla_decode_split_kernel(
   }
 }
 
+// Four partial values of a lane, bf16 or fp32
+__device__ __forceinline__ void store_part(uint16_t* p, f32x4_t v) {
+  *reinterpret_cast<uint2*>(p) = uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[0], v[1]}, bf16x2_t)),
+                                       __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[2], v[3]}, bf16x2_t))};
+}
+__device__ __forceinline__ void store_part(float* p, f32x4_t v) { *reinterpret_cast<f32x4_t*>(p) = v; }
+__device__ __forceinline__ f32x4_t part_value(uint2 raw) {
+  return f32x4_t{__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u), __uint_as_float(raw.y << 16),
+                 __uint_as_float(raw.y & 0xFFFF0000u)};
+}
+__device__ __forceinline__ f32x4_t part_value(f32x4_t raw) { return raw; }
+template <typename TP>
+struct MlaPart;  // a lane's load of four partial values
+template <>
+struct MlaPart<uint16_t> {
+  typedef uint2 vec;
+};
+template <>
+struct MlaPart<float> {
+  typedef f32x4_t vec;
+};
+
 // A split of at most 128 selected tokens of one row and 64 heads over an FP8
 // cache, all tokens at once: decode calls of a few rows are bound by the chain
 // of latencies of a split (ids, gather, conversion, scores, softmax, values),
@@ -1648,12 +1671,16 @@ __global__ void __launch_bounds__(256) mla_decode_split_kernel(
 //     probabilities go to LDS over the rope rows, which are no longer needed;
 //   * wave w multiplies all heads into columns 64 w .. + 63, V read out of the
 //     latent rows with transposing reads.
-// Partials are laid out as the block kernel's.  q goes through LDS first (its
+// Partials are laid out as the block kernel's, in fp32 up to kMdF32Chunks splits:
+// a row of few large splits averages their bf16 roundings less than the block
+// kernel's many small ones (512 picks, relative error against 64 bits: 2.4e-3 on
+// the block kernel, 2.5e-3 with bf16 partials here).  q goes through LDS first (its
 // fragments straight from memory cost 36 scattered loads a wave, 8 us of the
 // chain).  Measured: 8 rows x 128 heads x 2048 picks 27.9 us on the block kernel,
 // ~17 here; what is left is the chain itself (~24,000 cycles: ids and q 9,000,
 // conversion 4,000, scores 3,400, softmax 2,300, values 2,700, stores 1,800).
 constexpr int kMdTokens = 128;
+constexpr int kMdF32Chunks = 8;      // up to this many splits store fp32 partials
 constexpr int kMdRow = kMlaDl + 8;   // bf16 per latent row in LDS
 constexpr int kMdRope = 64 + 8;      // bf16 per rope row
 constexpr int kMdPs = kMdTokens + 8; // bf16 per row of P
@@ -1661,10 +1688,11 @@ static_assert(64 * kMdPs <= kMdTokens * kMdRope, "P overlays the rope rows");
 constexpr int kMdQCopies = 64 * (kMlaDl + 64) * 2 / 1024 / 8;  // 1 KB copies of q a wave
 static_assert(64 * (kMlaDl + 64) <= kMdTokens * kMdRow, "q is staged where the latent rows go");
 
+template <typename TP>
 __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* __restrict__ q, const MlaKv kv,
                                                                const int32_t* __restrict__ idx,
-                                                               uint16_t* __restrict__ part_o,
-                                                               float* __restrict__ part_ml, int topk, float scale) {
+                                                               TP* __restrict__ part_o, float* __restrict__ part_ml,
+                                                               int topk, float scale) {
   constexpr int DQK = kMlaDl + 64, NS = DQK / 32, NSL = kMlaDl / 32;
   __shared__ __attribute__((aligned(16))) uint16_t Kt[kMdTokens * kMdRow];
   __shared__ __attribute__((aligned(16))) uint16_t Rp[kMdTokens * kMdRope];
@@ -1880,16 +1908,12 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
 #pragma unroll
       for (int ht = 0; ht < 4; ++ht) o[ht][dl] = mfma_bf16(pa[ht], vv[dl], o[ht][dl]);
   }
-  uint16_t* po = part_o + ((int64_t)b * S + split) * (H / 16) * (kMlaDt * 256);
+  TP* po = part_o + ((int64_t)b * S + split) * (H / 16) * (kMlaDt * 256);
 #pragma unroll
   for (int ht = 0; ht < 4; ++ht)
 #pragma unroll
-    for (int dl = 0; dl < 4; ++dl) {
-      const f32x4_t v = o[ht][dl];
-      *reinterpret_cast<uint2*>(po + (((int64_t)(4 * blockIdx.z + ht) * kMlaDt + 4 * wv + dl) * 64 + lane) * 4) =
-          uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[0], v[1]}, bf16x2_t)),
-                __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{v[2], v[3]}, bf16x2_t))};
-    }
+    for (int dl = 0; dl < 4; ++dl)
+      store_part(po + (((int64_t)(4 * blockIdx.z + ht) * kMlaDt + 4 * wv + dl) * 64 + lane) * 4, o[ht][dl]);
   if (tid < 64) {
     const float m = fmaxf(fmaxf(Mx[0][tid], Mx[1][tid]), fmaxf(Mx[2][tid], Mx[3][tid]));
     const float l = (Lx[0][tid] + Lx[1][tid]) + (Lx[2][tid] + Lx[3][tid]);
@@ -1902,7 +1926,8 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
 // term and normalize.  Each wave turns the split maxima/sums of four heads
 // into weights (lane = split); then wave w blends splits w, w + 4, ... of the
 // tile's 64 x 4 partial values, and wave 0 sums the four and writes bf16.
-__global__ void __launch_bounds__(256) mla_combine_kernel(const uint16_t* __restrict__ part_o,
+template <typename TP>
+__global__ void __launch_bounds__(256) mla_combine_kernel(const TP* __restrict__ part_o,
                                                           const float* __restrict__ part_ml,
                                                           const float* __restrict__ sink, uint16_t* __restrict__ out,
                                                           int H, int S) {
@@ -1925,13 +1950,11 @@ __global__ void __launch_bounds__(256) mla_combine_kernel(const uint16_t* __rest
   __syncthreads();
   const int hq = lane >> 4;  // rows 4 hq + r of the tile
   const int64_t sstride = (int64_t)(H / 16) * kMlaDt * 256;
-  const uint16_t* po = part_o + (int64_t)b * S * sstride + ((int64_t)ht * kMlaDt + dt) * 256 + lane * 4;
+  const TP* po = part_o + (int64_t)b * S * sstride + ((int64_t)ht * kMlaDt + dt) * 256 + lane * 4;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = wv; s < S; s += 4) {
-    const uint2 raw = *reinterpret_cast<const uint2*>(po + s * sstride);
-    const float v[4] = {__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
-                        __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u)};
+    const f32x4_t v = part_value(*reinterpret_cast<const typename MlaPart<TP>::vec*>(po + s * sstride));
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] += wgt[s][4 * hq + r] * v[r];
   }
@@ -1954,7 +1977,8 @@ __global__ void __launch_bounds__(256) mla_combine_kernel(const uint16_t* __rest
 // slower, 19.5 against 17.5 us).
 constexpr int kMlaCombineTiles = 4;  // 16-column tiles a workgroup
 
-__global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const uint16_t* __restrict__ part_o,
+template <typename TP>
+__global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const TP* __restrict__ part_o,
                                                           const float* __restrict__ part_ml,
                                                           const float* __restrict__ sink, uint16_t* __restrict__ out,
                                                           int H, int S) {
@@ -1964,13 +1988,14 @@ __global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const uint16_t* 
   const int dt = blockIdx.x * kMlaCombineTiles + wv;
   const int hq = lane >> 4;  // rows 4 hq + r of the tile
   const int64_t sstride = (int64_t)(H / 16) * kMlaDt * 256;
-  const uint16_t* po = part_o + (int64_t)b * S * sstride + ((int64_t)ht * kMlaDt + dt) * 256 + lane * 4;
-  constexpr int CH = 32;
-  uint2 raw[CH];
+  const TP* po = part_o + (int64_t)b * S * sstride + ((int64_t)ht * kMlaDt + dt) * 256 + lane * 4;
+  typedef typename MlaPart<TP>::vec vec_t;
+  constexpr int CH = sizeof(TP) == 2 ? 32 : kMdF32Chunks;
+  vec_t raw[CH];
   auto load_chunk = [&](int s0) {
 #pragma unroll
     for (int i = 0; i < CH; ++i)
-      raw[i] = s0 + i < S ? *reinterpret_cast<const uint2*>(po + (s0 + i) * sstride) : make_uint2(0u, 0u);
+      raw[i] = s0 + i < S ? *reinterpret_cast<const vec_t*>(po + (s0 + i) * sstride) : vec_t{};
   };
   load_chunk(0);
 #pragma unroll
@@ -1992,8 +2017,7 @@ __global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const uint16_t* 
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       if (s0 + i < S) {
-        const float v[4] = {__uint_as_float(raw[i].x << 16), __uint_as_float(raw[i].x & 0xFFFF0000u),
-                            __uint_as_float(raw[i].y << 16), __uint_as_float(raw[i].y & 0xFFFF0000u)};
+        const f32x4_t v = part_value(raw[i]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] += wgt[s0 + i][4 * hq + r] * v[r];
       }
@@ -2585,7 +2609,8 @@ static int mla_chunks(int64_t b, int64_t h, int64_t topk) {
   return h % 64 == 0 && chunks <= 32 && b <= 32 && wgs >= 24 && wgs <= 1024 ? (int)chunks : 0;
 }
 static size_t mla_ws(int64_t b, int64_t h, int64_t topk, char* base, MlaWs* w) {
-  const int64_t S = std::max(mla_splits(b, topk), mla_chunks(b, h, topk));
+  const int64_t chunks = mla_chunks(b, h, topk);
+  const int64_t S = std::max<int64_t>(mla_splits(b, topk), chunks <= kMdF32Chunks ? 2 * chunks : chunks);
   const size_t ob = align256((size_t)b * S * h * kMlaDl * 2);
   const size_t mb = align256((size_t)b * S * h * 2 * 4);
   if (w) {
@@ -2717,10 +2742,16 @@ static int launch_mla(const uint16_t* q, const MlaKv& kv, const float* sink, con
   mla_ws(rows, h, topk, (char*)workspace, &ws);
   int S = mla_splits(rows, topk);
   const int chunks = FP8 && kv.n > 0 ? mla_chunks(rows, h, topk) : 0;
+  const bool f32 = chunks > 0 && chunks <= kMdF32Chunks;
   if (chunks > 0) {
     S = chunks;
-    MOSAIC_LAUNCH(mla_decode_chunk_kernel, dim3((unsigned)S, (unsigned)rows, (unsigned)(h / 64)), dim3(512), 0, st, q,
-                  kv, idx, ws.part_o, ws.part_ml, (int)topk, softmax_scale);
+    const dim3 grid((unsigned)S, (unsigned)rows, (unsigned)(h / 64));
+    if (f32)
+      MOSAIC_LAUNCH(mla_decode_chunk_kernel<float>, grid, dim3(512), 0, st, q, kv, idx,
+                    reinterpret_cast<float*>(ws.part_o), ws.part_ml, (int)topk, softmax_scale);
+    else
+      MOSAIC_LAUNCH(mla_decode_chunk_kernel<uint16_t>, grid, dim3(512), 0, st, q, kv, idx, ws.part_o, ws.part_ml,
+                    (int)topk, softmax_scale);
     MOSAIC_LAUNCH_CHECK("mla_decode_chunk");
   } else {
     const int blocks = (int)((topk + kMlaBT - 1) / kMlaBT);
@@ -2738,13 +2769,20 @@ static int launch_mla(const uint16_t* q, const MlaKv& kv, const float* sink, con
     }
     MOSAIC_LAUNCH_CHECK("mla_decode_split");
   }
-  if (rows * (h / 16) * (kMlaDt / kMlaCombineTiles) >= 256)
-    MOSAIC_LAUNCH(mla_combine_tiles_kernel,
-                  dim3((unsigned)(kMlaDt / kMlaCombineTiles), (unsigned)(h / 16), (unsigned)rows), dim3(256), 0, st,
-                  ws.part_o, ws.part_ml, sink, out, (int)h, S);
+  auto combine = [&](auto* part) {
+    using TP = std::remove_pointer_t<decltype(part)>;
+    if (rows * (h / 16) * (kMlaDt / kMlaCombineTiles) >= 256)
+      MOSAIC_LAUNCH(mla_combine_tiles_kernel<TP>,
+                    dim3((unsigned)(kMlaDt / kMlaCombineTiles), (unsigned)(h / 16), (unsigned)rows), dim3(256), 0, st,
+                    part, ws.part_ml, sink, out, (int)h, S);
+    else
+      MOSAIC_LAUNCH(mla_combine_kernel<TP>, dim3((unsigned)kMlaDt, (unsigned)(h / 16), (unsigned)rows), dim3(256), 0,
+                    st, part, ws.part_ml, sink, out, (int)h, S);
+  };
+  if (f32)
+    combine(reinterpret_cast<float*>(ws.part_o));
   else
-    MOSAIC_LAUNCH(mla_combine_kernel, dim3((unsigned)kMlaDt, (unsigned)(h / 16), (unsigned)rows), dim3(256), 0, st,
-                  ws.part_o, ws.part_ml, sink, out, (int)h, S);
+    combine(ws.part_o);
   MOSAIC_RETURN_LAUNCH("mla_sparse_decode");
 }
 
