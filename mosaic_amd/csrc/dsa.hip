@@ -2608,8 +2608,10 @@ static int mla_chunks(int64_t b, int64_t h, int64_t topk) {
   const int64_t wgs = b * (h / 64) * chunks;
   return h % 64 == 0 && chunks <= 32 && b <= 32 && wgs >= 24 && wgs <= 1024 ? (int)chunks : 0;
 }
-static size_t mla_ws(int64_t b, int64_t h, int64_t topk, char* base, MlaWs* w) {
-  const int64_t chunks = mla_chunks(b, h, topk);
+// `chunks`: splits of the whole-split kernel, 0 for the block kernel.  Queries
+// ask for the larger of both; a call with room for the block kernel's partials
+// only (a workspace sized for the bf16 cache, or for another batch) runs that.
+static size_t mla_ws(int64_t b, int64_t h, int64_t topk, int64_t chunks, char* base, MlaWs* w) {
   const int64_t S = std::max<int64_t>(mla_splits(b, topk), chunks <= kMdF32Chunks ? 2 * chunks : chunks);
   const size_t ob = align256((size_t)b * S * h * kMlaDl * 2);
   const size_t mb = align256((size_t)b * S * h * 2 * 4);
@@ -2730,18 +2732,20 @@ extern "C" int mosaic_dsa_indexer_bounds(const uint8_t* q, const float* q_s, con
 
 extern "C" size_t mosaic_mla_decode_workspace_bytes(int64_t b, int64_t h, int64_t topk) {
   if (b < 0 || h < 0 || topk < 0) return 0;
-  return mla_ws(b, h, topk, nullptr, nullptr);
+  return mla_ws(b, h, topk, mla_chunks(b, h, topk), nullptr, nullptr);
 }
 
 namespace mosaic {
 
 template <bool FP8, int DR>
 static int launch_mla(const uint16_t* q, const MlaKv& kv, const float* sink, const int32_t* idx, uint16_t* out,
-                      int64_t rows, int64_t h, int64_t topk, float softmax_scale, void* workspace, hipStream_t st) {
+                      int64_t rows, int64_t h, int64_t topk, float softmax_scale, void* workspace, size_t workspace_bytes,
+                      hipStream_t st) {
   MlaWs ws;
-  mla_ws(rows, h, topk, (char*)workspace, &ws);
   int S = mla_splits(rows, topk);
-  const int chunks = FP8 && kv.n > 0 ? mla_chunks(rows, h, topk) : 0;
+  int chunks = FP8 && kv.n > 0 ? mla_chunks(rows, h, topk) : 0;
+  if (mla_ws(rows, h, topk, chunks, nullptr, nullptr) > workspace_bytes) chunks = 0;
+  mla_ws(rows, h, topk, chunks, (char*)workspace, &ws);
   const bool f32 = chunks > 0 && chunks <= kMdF32Chunks;
   if (chunks > 0) {
     S = chunks;
@@ -2795,7 +2799,7 @@ static int check_mla_common(int64_t rows, int64_t h, int64_t n, int64_t topk, in
                    "mla_sparse_decode: shape out of range (topk at most %d)", kMlaMaxSplits * kMlaMaxChunk);
   MOSAIC_CHECK_ARG(rows_per_kv >= 1 && rows % rows_per_kv == 0, "mla_sparse_decode: rows %lld, rows_per_kv %lld",
                    (long long)rows, (long long)rows_per_kv);
-  const size_t need = mla_ws(rows, h, topk, nullptr, nullptr);
+  const size_t need = mla_ws(rows, h, topk, 0, nullptr, nullptr);
   MOSAIC_CHECK_ARG(workspace && workspace_bytes >= need, "mla_sparse_decode: workspace %zu bytes < %zu",
                    workspace_bytes, need);
   return kOk;
@@ -2820,7 +2824,8 @@ extern "C" int mosaic_mla_sparse_decode(const uint16_t* q, const uint8_t* kv_lat
   if (rc) return rc;
   if (b == 0) return kOk;
   const MlaKv kv{kv_latent, kv_scale, kv_rope, n, 1, sb_shift};
-  return launch_mla<true, 64>(q, kv, sink, idx, out, b, h, topk, softmax_scale, workspace, (hipStream_t)stream);
+  return launch_mla<true, 64>(q, kv, sink, idx, out, b, h, topk, softmax_scale, workspace, workspace_bytes,
+                              (hipStream_t)stream);
 }
 
 extern "C" int mosaic_mla_sparse_decode_bf16(const uint16_t* q, const uint16_t* kv, const float* sink,
@@ -2855,6 +2860,8 @@ extern "C" int mosaic_mla_sparse_decode_bf16(const uint16_t* q, const uint16_t* 
   }
   const MlaKv kvd{kv, nullptr, nullptr, n, (int)rows_per_kv, 0};
   if (d == 576)
-    return launch_mla<false, 64>(q, kvd, sink, idx, out, rows, h, topk, softmax_scale, workspace, (hipStream_t)stream);
-  return launch_mla<false, 0>(q, kvd, sink, idx, out, rows, h, topk, softmax_scale, workspace, (hipStream_t)stream);
+    return launch_mla<false, 64>(q, kvd, sink, idx, out, rows, h, topk, softmax_scale, workspace, workspace_bytes,
+                                 (hipStream_t)stream);
+  return launch_mla<false, 0>(q, kvd, sink, idx, out, rows, h, topk, softmax_scale, workspace, workspace_bytes,
+                              (hipStream_t)stream);
 }

@@ -254,6 +254,31 @@ def test_mla_fp8_whole_splits_vs_oracle(dev, b, h, n, t, sb, masked):
     _close(out.float().cpu().numpy(), D.mla_sparse_decode(q, lat, ls, rope, snk, idx, 0.06, sb))
 
 
+@pytest.mark.parametrize("b,h,t", [(24, 128, 1000), (12, 64, 2048)])
+def test_mla_fp8_block_kernel_workspace(dev, b, h, t):
+    """A workspace with room for the block kernel's partials only is taken, not refused, and nothing past it
+    is written; one byte less is refused."""
+    from mosaic_amd import _lib, ops
+    rng = np.random.default_rng(b + t)
+    q, lat, ls, rope, idx = _mla(rng, b, h, 2100, t, 64, 0.2)
+    size = _lib.lib().mosaic_mla_decode_workspace_bytes
+    splits = size(b, 16, t) // (b * 16 * 1024)  # 16 heads never take the whole-split kernel
+    need = b * splits * h * (1024 + 8)
+    assert need < size(b, h, t)
+    qd, latd, lsd, rd, idxd = _t(dev, q, lat, ls, rope, idx)
+    qd, rd = qd.to(torch.bfloat16), rd.to(torch.bfloat16)
+    ws = torch.full((size(b, h, t),), 0xA5, dtype=torch.uint8, device=dev)
+    out = torch.empty(b, h, 512, dtype=torch.bfloat16, device=dev)
+    run = lambda n: _lib.call("mosaic_mla_sparse_decode", qd.data_ptr(), latd.data_ptr(), lsd.data_ptr(),
+                              rd.data_ptr(), None, idxd.data_ptr(), out.data_ptr(), b, h, 2100, t, 512, 64, 64, 0.06,
+                              ws.data_ptr(), n, ops._stream())
+    run(need)
+    _close(out.float().cpu().numpy(), D.mla_sparse_decode(q, lat, ls, rope, None, idx, 0.06, 64))
+    assert bool((ws[need:] == 0xA5).all())
+    with pytest.raises(Exception, match="workspace"):
+        run(need - 1)
+
+
 def test_mla_wide_score_range(dev):
     """Scores rising by over a hundred nats along the token order (the rope part
     grows 300-fold): every head's running maximum moves past the lazy margin
