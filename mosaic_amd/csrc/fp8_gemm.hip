@@ -1102,7 +1102,9 @@ static float fp8_tiled_time(int kind, int S, int64_t m, int64_t n, int64_t k) {
   const float t = fixed + (float)((wgs + 255) / 256) * (round + step * (float)steps);
   return slices == 1 ? t : t + 2.f + 8.f * (float)slices * (float)m * (float)n / 5.5e6f;
 }
-static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k) {
+// `max_splits` is 1 for a call without room for partials: the best kernel that
+// does not split.
+static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, int max_splits = 8) {
   const int64_t nkb = k / 128;
   // Tiled kernels from 96 rows; at 65..95 rows for weights of 8 MB and more (18432
   // x 7168: 180 -> 46 us; 576 x 7168: the skinny kernel's 11.7 against 14.5 us).
@@ -1113,7 +1115,7 @@ static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k) {
     for (int kind = 1; kind <= (m > 128 ? 3 : 1); ++kind) {
       // the 256 x 256 kernel addresses A and B with 32-bit offsets and does not split K
       if (kind == 3 && (m * k >= (1ll << 32) || n * k >= (1ll << 32))) continue;
-      for (int S = 1; S <= (kind == 3 ? 1 : 8) && (S == 1 || nkb / S >= 4); ++S) {
+      for (int S = 1; S <= (kind == 3 ? 1 : max_splits) && (S == 1 || nkb / S >= 4); ++S) {
         const float t = fp8_tiled_time(kind, S, m, n, k);
         if (best_t == 0.f || t < best_t) best = Fp8Plan{kind, S}, best_t = t;
       }
@@ -1131,7 +1133,7 @@ static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k) {
   // for weights of 8 MB and more (18432 x 7168, M = 64: 147 -> 61 us); below, the
   // skinny kernel's latency is lower (576 x 7168, M = 64: 12.1 against 13.6 us)
   if (m > 16 && m <= 64 && n % 16 == 0 && n * k >= (8ll << 20) && n * k < (1ll << 31))
-    return {5, fp8_mid_plan(m, n, k).S};
+    return {5, std::min(max_splits, fp8_mid_plan(m, n, k).S)};
   return {0, 1};
 }
 
@@ -1154,8 +1156,8 @@ static int fp8_block_gemm_impl(const uint8_t* a, const float* a_s, const uint8_t
   const int f32 = out_dtype == MOSAIC_DTYPE_F32;
   Fp8Plan plan = fp8_plan(m, n, k);
   if (plan.S > 1 && (!workspace || workspace_bytes < (size_t)plan.S * m * n * 4)) {
-    // no partials workspace: the whole K in one slice (the kernels of the plan without split)
-    plan = plan.kind == 1 && ((m + 127) / 128) * ((n + 127) / 128) < 32 ? Fp8Plan{0, 1} : Fp8Plan{plan.kind, 1};
+    // no partials workspace: the whole K in one slice
+    plan = fp8_plan(m, n, k, 1);
   }
   float* part = reinterpret_cast<float*>(workspace);
   const int64_t mt = (m + 15) / 16;

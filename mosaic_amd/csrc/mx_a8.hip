@@ -1081,7 +1081,9 @@ static float dense_a8_time(const DenseA8Plan& p, int64_t m, int64_t n, int64_t k
                              : 5.f + rounds * (5.f + (rows <= 128 ? 1.02f : rows <= 192 ? 1.1f : 1.54f) * steps);
   return p.splits == 1 ? t : t + 2.f + 8.f * (float)p.splits * (float)m * (float)n / 5.5e6f;
 }
-static DenseA8Plan dense_a8_plan(int64_t m, int64_t n, int64_t k) {
+// `max_splits` is 1 for a call without room for partials: the tile is then the
+// best unsplit one, not that of a split plan run unsplit.
+static DenseA8Plan dense_a8_plan(int64_t m, int64_t n, int64_t k, int max_splits = 8) {
   DenseA8Plan best{};
   float best_t = 0.f;
   for (int tr = m <= 2048 ? 64 : 256; tr <= 256; tr += 192) {  // (64-row tiles measured up to 2048 rows)
@@ -1090,7 +1092,7 @@ static DenseA8Plan dense_a8_plan(int64_t m, int64_t n, int64_t k) {
     p.n_row = (int)((m + tr - 1) / tr);
     p.n_col = (int)((n + 255) / 256);
     p.row_fastest = tr == 64 ? 1 : 0;
-    for (p.splits = 1; p.splits <= (int)std::min<int64_t>(8, k / 512); ++p.splits) {
+    for (p.splits = 1; p.splits <= (int)std::min<int64_t>(max_splits, k / 512); ++p.splits) {
       const float t = dense_a8_time(p, m, n, k);
       if (best_t == 0.f || t < best_t) best = p, best_t = t;
     }
@@ -1164,7 +1166,7 @@ static int mxt16_linear_a8_impl(const uint8_t* xq, const float* sa, const uint8_
       if (workspace && workspace_bytes >= dense_a8_ws_bytes(m, n, k))
         part = (float*)workspace;
       else
-        plan.splits = 1;  // no workspace: the unsplit plan
+        plan = dense_a8_plan(m, n, k, 1);
     }
     const int nwork = plan.n_row * plan.n_col * plan.splits;
     const int per_xcd = (nwork + 7) / 8;

@@ -88,6 +88,23 @@ def test_fp8_block_gemm_estimated_plans(dev, m, n, k, out):
     assert err.max() <= 2e-2, f"max scaled err {err.max()}"
 
 
+@pytest.mark.parametrize("m,n,k", [(48, 4096, 2048), (70, 2048, 4096), (200, 4112, 4096), (300, 1536, 3584),
+                                   (520, 1040, 4096)])
+def test_fp8_block_gemm_without_workspace(dev, m, n, k):
+    """A shape whose plan splits K, through the entry without a workspace: the best unsplit kernel."""
+    from mosaic_amd import _lib, ops
+    assert _lib.lib().mosaic_fp8_block_gemm_workspace_bytes(m, n, k) > 0
+    rng = np.random.default_rng(m + n + k)
+    aq, a_s, bq, bs = _case(rng, m, n, k)
+    t = [torch.from_numpy(np.ascontiguousarray(v)).to(dev) for v in (aq, a_s, bq, bs)]
+    c = torch.empty(m, n, dtype=torch.bfloat16, device=dev)
+    _lib.call("mosaic_fp8_block_gemm", *(v.data_ptr() for v in t), c.data_ptr(), ops.DT_BF16, m, n, k, ops._stream())
+    rows = np.unique(np.r_[0, 1, 15, m // 2, m - 2, m - 1, rng.integers(0, m, 8)])
+    ref = L.fp8_block_gemm(aq[rows], a_s[rows], bq, bs, out_bf16=True)
+    err = np.abs(c.float().cpu().numpy()[rows] - ref) / np.maximum(1.0, np.abs(ref))
+    assert err.max() <= 2e-2, f"max scaled err {err.max()}"
+
+
 @pytest.mark.parametrize("m,n,k,e8m0", [(1, 1536, 7168, False), (1, 18432, 7168, True), (16, 576, 7168, False),
                                         (37, 200, 1024, True), (80, 4096, 512, False), (3, 24576, 1536, True),
                                         (5, 16, 128, False),
