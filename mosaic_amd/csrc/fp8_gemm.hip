@@ -1090,6 +1090,13 @@ struct Fp8Plan {
 // them but 96 x 4096 x 4096, and 1.13x faster on average than the rule by tile
 // counts before (us, before / now: 300 x 18432 x 7168 143.8 / 92.1, 512 rows 159.5
 // / 109.6, 2048 x 7168 x 16384 342 / 227, 256 x 576 x 7168 21.1 / 16.8).
+// A single 256-row tile has a step of its own: with few workgroups its weight
+// stream is all of the time, with many the stream's rate (56 workgroups 0.73 us a
+// K block, 128 0.71, 144 1.08, 192 1.05).  One step for all row counts split 200 x
+// 18432 x 7168 three ways at 73.9 us where the whole K takes 64.1 (205 x 21584 x
+// 11264 106.8 / 99.8, 171 x 23312 x 15232 150.1 / 138.4), and left 245 x 11680 x
+// 10112 on 128-row tiles (66.7 / 61.8); of 14 shapes whose plan moved, 136 x 5696 x
+// 6656 alone lost (25.7 / 26.1).
 static float fp8_tiled_time(int kind, int S, int64_t m, int64_t n, int64_t k) {
   const int64_t bm = kind == 1 ? 128 : 256, bn = kind == 3 ? 256 : 128, nkb = k / 128;
   const int64_t steps = (nkb + S - 1) / S, slices = (nkb + steps - 1) / steps, n_row = (m + bm - 1) / bm;
@@ -1097,7 +1104,7 @@ static float fp8_tiled_time(int kind, int S, int64_t m, int64_t n, int64_t k) {
   const float streams = (float)std::min<int64_t>(256, wgs) / (256.f * (float)n_row);
   const float fixed = kind == 1 ? 4.f : kind == 2 ? 5.f : 6.f, round = kind == 3 ? 4.f : 1.f;
   const float step = kind == 1   ? 0.68f + 0.30f * streams
-                     : kind == 2 ? 1.20f + 0.25f * streams
+                     : kind == 2 ? (n_row == 1 ? 0.65f + 0.80f * streams : 1.20f + 0.25f * streams)
                                  : 1.65f + 0.35f * streams;
   const float t = fixed + (float)((wgs + 255) / 256) * (round + step * (float)steps);
   return slices == 1 ? t : t + 2.f + 8.f * (float)slices * (float)m * (float)n / 5.5e6f;

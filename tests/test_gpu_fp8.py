@@ -71,6 +71,8 @@ def test_fp8_block_gemm_vs_oracle(dev, m, n, k, out):
 @pytest.mark.parametrize("m,n,k", [
     # 256-row tiles from 129 rows (ragged M and N, two rounds of workgroups, one and two K blocks a stage ring)
     (129, 33000, 128), (200, 24592, 256), (255, 20000, 1024), (500, 9000, 640),
+    # one 256-row tile: whole, and split 2 and 5 ways
+    (169, 17776, 7168), (150, 11680, 10112), (239, 6288, 8320),
     # 128-row tiles above 256 rows, unsplit and split 8, 7 and 2 ways (N % 4 != 0: the scalar reduce)
     (257, 576, 4096), (300, 1536, 3584), (321, 2050, 1024), (770, 1030, 1024), (300, 18448, 512),
     # the 256 x 256 kernel on fewer than 256 tiles, ragged
