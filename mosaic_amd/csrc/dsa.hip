@@ -2743,7 +2743,8 @@ static int launch_mla(const uint16_t* q, const MlaKv& kv, const float* sink, con
                       hipStream_t st) {
   MlaWs ws;
   int S = mla_splits(rows, topk);
-  int chunks = FP8 && kv.n > 0 ? mla_chunks(rows, h, topk) : 0;
+  // (q goes straight into LDS there, 16 bytes a lane: other alignments keep the block kernel's register loads)
+  int chunks = FP8 && kv.n > 0 && (uintptr_t)q % 16 == 0 ? mla_chunks(rows, h, topk) : 0;
   if (mla_ws(rows, h, topk, chunks, nullptr, nullptr) > workspace_bytes) chunks = 0;
   mla_ws(rows, h, topk, chunks, (char*)workspace, &ws);
   const bool f32 = chunks > 0 && chunks <= kMdF32Chunks;
@@ -2840,8 +2841,11 @@ extern "C" int mosaic_mla_sparse_decode_bf16(const uint16_t* q, const uint16_t* 
   // From 64 rows the row kernel: splitting a row over workgroups no longer pays
   // for its partials and combine (64 heads, us, split path against rows: 32 rows
   // of 640 picks 27.1 / 32.3, 64 rows 40.1 / 33.6, 64 rows of 2048 picks 86.1 /
-  // 82.5, 128 rows 112.7 / 83.7; 16 heads, 64 rows of 640 30.6 / 24.6).
-  if (d == 512 && topk <= kMrMaxPicks && rows >= kMrMinRows) {
+  // 82.5, 128 rows 112.7 / 83.7; 16 heads, 64 rows of 640 30.6 / 24.6).  It copies
+  // the cache's rows straight into LDS, 16 bytes a lane, and stores 16 bytes: rows
+  // that are not aligned for that keep the split kernel's register loads.
+  const bool aligned = ((uintptr_t)q | (uintptr_t)kv | (uintptr_t)out) % 16 == 0;
+  if (d == 512 && topk <= kMrMaxPicks && rows >= kMrMinRows && aligned) {
     int ht = 4;
     while (ht > 1 && (h / 16) % ht != 0) --ht;
     const int groups = (int)(h / (16 * ht));

@@ -279,6 +279,57 @@ def test_mla_fp8_block_kernel_workspace(dev, b, h, t):
         run(need - 1)
 
 
+def _skewed(a, dev):
+    """bf16 copy of a whose first element lies 4 bytes past a 16-byte boundary"""
+    t = torch.from_numpy(a)
+    return torch.empty(a.size + 2, dtype=torch.bfloat16, device=dev)[2:].view(a.shape).copy_(t)
+
+
+def test_mla_fp8_unaligned_q_keeps_block_kernel(dev):
+    """A q that is not 16-byte aligned never reaches the kernel that copies q straight into LDS: bit for bit
+    the block kernel's result, which a workspace with room for its partials only asks for."""
+    from mosaic_amd import _lib, ops
+    b, h, n, t = 12, 64, 1100, 1000
+    rng = np.random.default_rng(11)
+    q, lat, ls, rope, idx = _mla(rng, b, h, n, t, 64, 0.2)
+    qd, latd, lsd, rd, idxd = _t(dev, q, lat, ls, rope, idx)
+    qd, rd, qs = qd.to(torch.bfloat16), rd.to(torch.bfloat16), _skewed(q, dev)
+    assert qd.data_ptr() % 16 == 0 and qs.data_ptr() % 16 == 4
+    size = _lib.lib().mosaic_mla_decode_workspace_bytes
+    block = b * (size(b, 16, t) // (b * 16 * 1024)) * h * (1024 + 8)
+    assert block < size(b, h, t)
+    ws = torch.empty(size(b, h, t), dtype=torch.uint8, device=dev)
+
+    def run(qt, nbytes):
+        out = torch.empty(b, h, 512, dtype=torch.bfloat16, device=dev)
+        _lib.call("mosaic_mla_sparse_decode", qt.data_ptr(), latd.data_ptr(), lsd.data_ptr(), rd.data_ptr(), None,
+                  idxd.data_ptr(), out.data_ptr(), b, h, n, t, 512, 64, 64, 0.06, ws.data_ptr(), nbytes,
+                  ops._stream())
+        return out
+
+    got = run(qs, size(b, h, t))
+    assert torch.equal(got, run(qd, block))
+    _close(got.float().cpu().numpy(), D.mla_sparse_decode(q, lat, ls, rope, None, idx, 0.06, 64))
+
+
+@pytest.mark.parametrize("skew", ["none", "q", "kv"])
+def test_mla_rows_bf16_unaligned_keeps_split_kernel(dev, skew):
+    """From 64 rows the row kernel (one launch) takes 16-byte aligned operands only; others keep the split
+    and combine kernels (two launches)."""
+    from mosaic_amd import _lib, ops
+    rows, h, n, t = 64, 16, 200, 65
+    rng = np.random.default_rng(5)
+    q = C.round_bf16(rng.standard_normal((rows, h, 512)).astype(np.float32))
+    kv = C.round_bf16(rng.standard_normal((1, n, 512)).astype(np.float32))
+    idx = rng.integers(0, n, (rows, t)).astype(np.int32)
+    place = lambda a, name: _skewed(a, dev) if skew == name else torch.from_numpy(a).to(dev).to(torch.bfloat16)
+    qd, kvd, idxd = place(q, "q"), place(kv, "kv"), torch.from_numpy(idx).to(dev)
+    before = _lib.lib().mosaic_launch_count()
+    out = ops.mla_sparse_decode_bf16(qd, kvd, idxd, 512 ** -0.5)
+    assert _lib.lib().mosaic_launch_count() - before == (1 if skew == "none" else 2)
+    _close(out.float().cpu().numpy(), D.sparse_attn(q, kv, None, idx, 512 ** -0.5, 512, rows))
+
+
 def test_mla_wide_score_range(dev):
     """Scores rising by over a hundred nats along the token order (the rope part
     grows 300-fold): every head's running maximum moves past the lazy margin
