@@ -1686,6 +1686,13 @@ constexpr int kMdRope = 64 + 8;      // bf16 per rope row
 constexpr int kMdPs = kMdTokens + 8; // bf16 per row of P
 static_assert(64 * kMdPs <= kMdTokens * kMdRope, "P overlays the rope rows");
 constexpr int kMdQCopies = 64 * (kMlaDl + 64) * 2 / 1024 / 8;  // 1 KB copies of q a wave
+constexpr int kMdLat = kMdTokens * kMlaDl / (512 * 16);        // latent pieces (16 bytes) a thread, each with its scale
+constexpr int kMdRopes = kMdTokens * 64 * 2 / (512 * 16);      // rope pieces (16 bytes) a thread
+// Vector loads a wave issues between q's copies and the wait for them.  Loads
+// complete in order, so at most this many in flight means that q has landed;
+// tests/test_codegen.py counts them in the built kernel (fewer, merged or moved
+// past the wait, would let waves read q's LDS early).
+constexpr int kMdGather = 2 * kMdLat + kMdRopes;
 static_assert(64 * (kMlaDl + 64) <= kMdTokens * kMdRow, "q is staged where the latent rows go");
 
 template <typename TP>
@@ -1725,22 +1732,22 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
   // by scalar loads, which do not wait for q's copies.
   const int32_t* ids = idx + (int64_t)b * topk + t0;
   const int lp = lane & 31, rp = lane & 7, lt = 2 * wv + (lane >> 5);
-  int id2[8][2];
+  int id2[kMdLat][2];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < kMdLat; ++i)
 #pragma unroll
     for (int u = 0; u < 2; ++u) id2[i][u] = ids[min(16 * i + 2 * wv + u, nt - 1)];
   __builtin_amdgcn_sched_barrier(0);  // all loads first: one wait instead of sixteen
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < kMdLat; ++i)
 #pragma unroll
     for (int u = 0; u < 2; ++u)  // (a negative id stays negative)
       id2[i][u] = 16 * i + 2 * wv + u < nt && (int64_t)id2[i][u] < n ? id2[i][u] : -1;
-  int lid[8], rid[2], rt[2];
+  int lid[kMdLat], rid[kMdRopes], rt[kMdRopes];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) lid[i] = lane < 32 ? id2[i][0] : id2[i][1];
+  for (int i = 0; i < kMdLat; ++i) lid[i] = lane < 32 ? id2[i][0] : id2[i][1];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < kMdRopes; ++j) {
     rid[j] = id2[4 * j][0];
 #pragma unroll
     for (int g = 1; g < 8; ++g) rid[j] = (lane >> 3) == g ? id2[4 * j + (g >> 1)][g & 1] : rid[j];
@@ -1748,21 +1755,21 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
   }
   // masked tokens read row 0 and are zeroed below (loads under a branch would be
   // waited for at its end)
-  u32x4_t raw[8], rope[2];
-  float sc[8];
+  u32x4_t raw[kMdLat], rope[kMdRopes];
+  float sc[kMdLat];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < kMdLat; ++i) {
     const int64_t r = kvb + max(lid[i], 0);
     raw[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(kv.lat) + r * kMlaDl + 16 * lp);
     sc[i] = kv.lat_s[r * nsc + ((16 * lp) >> kv.sb_shift)];
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < kMdRopes; ++i) {
     rope[i] = *reinterpret_cast<const u32x4_t*>(kv.rope + (kvb + max(rid[i], 0)) * 64 + 8 * rp);
   }
   // q has landed (the gather may still fly); it becomes the B operand of S^T:
   // heads 32 hh + 16 t + c of the group
-  asm volatile("s_waitcnt vmcnt(18)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kMdGather) : "memory");
   bf16x8_t qf[2][NS];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -1774,10 +1781,10 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // q's LDS may be overwritten
   if (lp == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) Live[16 * i + lt] = lid[i] >= 0 ? 1 : 0;
+    for (int i = 0; i < kMdLat; ++i) Live[16 * i + lt] = lid[i] >= 0 ? 1 : 0;
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < kMdLat; ++i) {
     uint32_t o[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1797,7 +1804,7 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
     dst[1] = ok ? u32x4_t{o[4], o[5], o[6], o[7]} : u32x4_t{0u, 0u, 0u, 0u};
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < kMdRopes; ++i) {
     *reinterpret_cast<u32x4_t*>(&Rp[rt[i] * kMdRope + 8 * rp]) = rid[i] >= 0 ? rope[i] : u32x4_t{0u, 0u, 0u, 0u};
   }
   __syncthreads();
