@@ -158,6 +158,12 @@ int mosaic_fp8_block_gemm(const uint8_t* a, const float* a_s, const uint8_t* b, 
  * fp8_gemm launches allocate nothing; it serves the same call sites. */
 size_t mosaic_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 
+/* The kernel those entries run for a shape, with or without room for partials:
+ * 256 * kind + K slices (kind 0: skinny, 1: 128-row tiles, 2: 256-row tiles, 3:
+ * 256 x 256 tiles, 4: decode ring, 5: mid; -1: not a shape they take).  Host
+ * only; lets tests and tuning name the kernel that a shape reaches. */
+int mosaic_fp8_block_gemm_plan(int64_t m, int64_t n, int64_t k, int with_workspace);
+
 /* mosaic_fp8_block_gemm with a caller-provided workspace of workspace_bytes
  * (>= mosaic_fp8_block_gemm_workspace_bytes(m, n, k) to split K; with less,
  * or NULL, it runs unsplit).  The slices' fp32 partials are summed in slice

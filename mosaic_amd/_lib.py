@@ -36,6 +36,7 @@ SIGNATURES: dict[str, tuple] = {
     "mosaic_mxt16_linear_a16": (c_int, [P, P, P, P, I64, I64, I64, P]),
     "mosaic_fp8_block_gemm": (c_int, [P, P, P, P, P, I, I64, I64, I64, P]),
     "mosaic_fp8_block_gemm_workspace_bytes": (c_size_t, [I64, I64, I64]),
+    "mosaic_fp8_block_gemm_plan": (c_int, [I64, I64, I64, I]),
     "mosaic_fp8_block_gemm_ws": (c_int, [P, P, P, P, P, I, I64, I64, I64, P, c_size_t, P]),
     "mosaic_fp8_t16_prepack": (c_int, [P, P, I64, I64, P]),
     "mosaic_fp8_t16_unpack": (c_int, [P, P, I64, I64, P]),

@@ -1127,8 +1127,13 @@ static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, int max_splits = 8) {
         if (best_t == 0.f || t < best_t) best = Fp8Plan{kind, S}, best_t = t;
       }
     }
+    // Below 256 rows a grid of fewer than 32 workgroups of 128 rows leaves the shape
+    // to the skinny kernel, whichever tile won the estimate: that kernel fills the
+    // chip (us, without a workspace, 256-row tiles against the skinny kernel: 200 x
+    // 576 x 7168 55.1 / 19.9, 130 x 512 x 16384 118.8 / 33.6, 255 x 768 x 7168 56.2 /
+    // 26.9, 143 x 272 x 13824 102.0 / 23.5).
     const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    if (m >= 256 || best.kind != 1 || tiles * best.S >= 32) return best;
+    if (m >= 256 || tiles * best.S >= 32) return best;
   }
   // decode shapes: the ring kernel for wide N, and for narrower N when K is deep
   // enough for its 8-wave split to leave each wave >= 4 blocks (M = 1 / 16,
@@ -1207,6 +1212,12 @@ extern "C" size_t mosaic_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, in
   if (m <= 0 || n <= 0 || k <= 0 || k % 128) return 0;
   const Fp8Plan plan = fp8_plan(m, n, k);
   return plan.S > 1 ? (size_t)plan.S * (size_t)m * (size_t)n * 4 : 0;
+}
+
+extern "C" int mosaic_fp8_block_gemm_plan(int64_t m, int64_t n, int64_t k, int with_workspace) {
+  if (m <= 0 || n <= 0 || k <= 0 || k % 128) return -1;
+  const Fp8Plan plan = fp8_plan(m, n, k, with_workspace ? 8 : 1);
+  return plan.kind * 256 + plan.S;
 }
 
 extern "C" int mosaic_fp8_block_gemm_ws(const uint8_t* a, const float* a_s, const uint8_t* b, const float* b_s,
