@@ -1131,9 +1131,13 @@ static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, int max_splits = 8) {
     // to the skinny kernel, whichever tile won the estimate: that kernel fills the
     // chip (us, without a workspace, 256-row tiles against the skinny kernel: 200 x
     // 576 x 7168 55.1 / 19.9, 130 x 512 x 16384 118.8 / 33.6, 255 x 768 x 7168 56.2 /
-    // 26.9, 143 x 272 x 13824 102.0 / 23.5).
+    // 26.9, 143 x 272 x 13824 102.0 / 23.5).  At 8 to 11 K blocks a whole K, where
+    // the estimate takes it by choice, counts as the two slices it beats (us, skinny
+    // against whole K: 255 x 1504 x 1024 13.6 / 9.6, 128 x 2224 x 1024 12.0 / 9.9, 247
+    // x 1808 x 1152 17.2 / 10.3).
     const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    if (m >= 256 || tiles * best.S >= 32) return best;
+    const int64_t slices = best.S == 1 && max_splits > 1 && nkb >= 8 && nkb < 12 ? 2 : best.S;
+    if (m >= 256 || tiles * slices >= 32) return best;
   }
   // decode shapes: the ring kernel for wide N, and for narrower N when K is deep
   // enough for its 8-wave split to leave each wave >= 4 blocks (M = 1 / 16,
@@ -1216,7 +1220,8 @@ extern "C" size_t mosaic_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, in
 
 extern "C" int mosaic_fp8_block_gemm_plan(int64_t m, int64_t n, int64_t k, int with_workspace) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 128) return -1;
-  const Fp8Plan plan = fp8_plan(m, n, k, with_workspace ? 8 : 1);
+  Fp8Plan plan = fp8_plan(m, n, k);
+  if (plan.S > 1 && !with_workspace) plan = fp8_plan(m, n, k, 1);
   return plan.kind * 256 + plan.S;
 }
 

@@ -11,15 +11,25 @@ def _fp8(m, n, k, workspace=True):
 
 
 @pytest.mark.parametrize("m,n,k", [(200, 576, 7168), (130, 512, 16384), (255, 768, 7168), (140, 256, 16384),
-                                   (143, 272, 13824), (150, 832, 8960)])
+                                   (143, 272, 13824), (150, 832, 8960), (130, 1152, 1280)])
 def test_fp8_narrow_weights_without_workspace_run_skinny(m, n, k):
     """129..255 rows of a narrow weight: tiled with K split where the partials have room, else the skinny
     kernel (256-row tiles would be a handful of workgroups)."""
     kind, splits = _fp8(m, n, k)
-    assert kind in (T128, T256) and splits >= 4
+    assert kind in (T128, T256) and splits >= 2
     assert _fp8(m, n, k, workspace=False) == (SKINNY, 1)
 
 
 @pytest.mark.parametrize("m,n,k", [(200, 4112, 4096), (250, 2048, 1024)])
 def test_fp8_wider_weights_without_workspace_stay_tiled(m, n, k):
     assert _fp8(m, n, k, workspace=False)[0] in (T128, T256)
+
+
+@pytest.mark.parametrize("m,n,k", [(255, 1504, 1024), (128, 2224, 1024), (99, 2944, 1024), (189, 1296, 1152),
+                                   (247, 1808, 1152)])
+def test_fp8_short_k_whole_plans_stay_tiled(m, n, k):
+    """8 to 11 K blocks over 16 to 31 tiles: the estimate takes the whole K in one slice, which the
+    small-grid rule must not take for a grid too small to tile."""
+    for workspace in (True, False):
+        kind, splits = _fp8(m, n, k, workspace)
+        assert kind in (T128, T256) and splits == 1
