@@ -1122,8 +1122,14 @@ static Fp8Plan fp8_plan(int64_t m, int64_t n, int64_t k, int max_splits = 8) {
     for (int kind = 1; kind <= (m > 128 ? 3 : 1); ++kind) {
       // the 256 x 256 kernel addresses A and B with 32-bit offsets and does not split K
       if (kind == 3 && (m * k >= (1ll << 32) || n * k >= (1ll << 32))) continue;
+      // With a tile for every CU it is the choice unless another plan is 4% better:
+      // within that the estimate does not tell them apart (us, 256 x 256 tiles against
+      // its pick: 4733 x 4352 x 4480 137.7 / 142.6, 2867 x 13920 x 384 44.8 / 47.8, 973
+      // x 17744 x 2688 87.7 / 91.1; past it the pick wins, 2119 x 7440 x 3840 121.0 /
+      // 99.4, 810 x 17344 x 1152 51.2 / 37.6).
+      const float margin = kind == 3 && m >= 256 && ((m + 255) / 256) * ((n + 255) / 256) >= 256 ? 0.96f : 1.f;
       for (int S = 1; S <= (kind == 3 ? 1 : max_splits) && (S == 1 || nkb / S >= 4); ++S) {
-        const float t = fp8_tiled_time(kind, S, m, n, k);
+        const float t = margin * fp8_tiled_time(kind, S, m, n, k);
         if (best_t == 0.f || t < best_t) best = Fp8Plan{kind, S}, best_t = t;
       }
     }

@@ -33,3 +33,11 @@ def test_fp8_short_k_whole_plans_stay_tiled(m, n, k):
     for workspace in (True, False):
         kind, splits = _fp8(m, n, k, workspace)
         assert kind in (T128, T256) and splits == 1
+
+
+@pytest.mark.parametrize("m,n,k,kind", [
+    (4733, 4352, 4480, BIG), (2867, 13920, 384, BIG), (973, 17744, 2688, BIG), (2580, 6880, 5376, BIG),
+    (4096, 18432, 7168, BIG), (2119, 7440, 3840, T128), (810, 17344, 1152, T128), (786, 20688, 512, T256)])
+def test_fp8_big_tiles_keep_near_ties(m, n, k, kind):
+    """The 256 x 256 kernel with a tile for every CU gives way only to a plan that is clearly better."""
+    assert _fp8(m, n, k) == (kind, 1)
