@@ -1072,14 +1072,21 @@ __global__ void __launch_bounds__(256) mx_gemm_a8_reduce_kernel(const float* __r
 // counting tiles alone: 193 x 18432 x 7168 64-row tiles in two rounds 77.1 us,
 // 256-row tiles split 3 ways in one 54.9; 512 x 1536 x 7168 256-row tiles split 8
 // ways 33.7, 64-row tiles split 5 ways 22.5; 768 x 4096 x 4096 41.1 / 27.1.
+// Two constants come from 75 shapes beside those: a 64-row round's fixed part at K =
+// 512 (436 x 18720 x 512 64-row tiles 21.2 us, 256-row tiles 19.0; 1393 x 15472 38.1
+// / 33.9), and the partials' rate past 1024 rows, without which the split there was
+// too coarse (6939 x 592 x 2560 whole 42.3 us, split 3 ways 35.9; 2265 x 832 x 3072
+// 32.6 / 29.5; 1855 x 2288 x 4096 44.7 / 42.3).
 static float dense_a8_time(const DenseA8Plan& p, int64_t m, int64_t n, int64_t k) {
   const int64_t rows = std::min<int64_t>(m, p.tr), nch = k / 512;
   const float steps = 4.f * (float)((nch + p.splits - 1) / p.splits);
   const float rounds = (float)(((int64_t)p.n_row * p.n_col * p.splits + 255) / 256);
   // a step's cost by the rows multiplied (256-row tiles: waves own 64-row quarters)
-  const float t = rows <= 64 ? 4.f + rounds * (1.f + (0.55f + 0.15f * (float)m / (64.f * p.n_row)) * steps)
+  const float t = rows <= 64 ? 4.f + rounds * (1.4f + (0.55f + 0.15f * (float)m / (64.f * p.n_row)) * steps)
                              : 5.f + rounds * (5.f + (rows <= 128 ? 1.02f : rows <= 192 ? 1.1f : 1.54f) * steps);
-  return p.splits == 1 ? t : t + 2.f + 8.f * (float)p.splits * (float)m * (float)n / 5.5e6f;
+  // (bytes a us of the partials: the larger sums keep more of the chip busy)
+  const float rate = m > 1024 ? 8e6f : 5.5e6f;
+  return p.splits == 1 ? t : t + 2.f + 8.f * (float)p.splits * (float)m * (float)n / rate;
 }
 // `max_splits` is 1 for a call without room for partials: the tile is then the
 // best unsplit one, not that of a split plan run unsplit.

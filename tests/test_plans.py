@@ -41,3 +41,11 @@ def test_fp8_short_k_whole_plans_stay_tiled(m, n, k):
 def test_fp8_big_tiles_keep_near_ties(m, n, k, kind):
     """The 256 x 256 kernel with a tile for every CU gives way only to a plan that is clearly better."""
     assert _fp8(m, n, k) == (kind, 1)
+
+
+@pytest.mark.parametrize("m,n,k,splits", [
+    (6939, 592, 2560, 3), (2265, 832, 3072, 6), (2243, 3520, 3072, 2), (2428, 1200, 2048, 4), (1855, 2288, 4096, 3),
+    (5220, 560, 1536, 3), (2763, 1808, 1024, 1), (193, 18432, 7168, 3), (512, 1536, 7168, 5), (768, 4096, 4096, 1)])
+def test_a8_splits(m, n, k, splits):
+    """K slices of the dense A8 GEMM, above the row count where the partials' rate changes and below."""
+    assert _lib.lib().mosaic_mxt16_linear_a8_workspace_bytes(m, n, k) == (4 * m * n * splits if splits > 1 else 0)
