@@ -934,8 +934,8 @@ __global__ void __launch_bounds__(1024) dsa_finish_kernel(const uint64_t* __rest
 // Indexer + exact top-k of many query rows that share short key caches (a
 // prompt: row t sees the first (t + 1) / ratio entries).  Picks are most of a
 // row's entries there, so bounding first would save little: every entry gets
-// its exact score, and the row's keys are sorted, in one kernel without a
-// workspace.
+// its exact score, and the row's keys are sorted, in one kernel that needs no
+// workspace (its callers give the certified path's, which it leaves alone).
 //
 // A workgroup takes kDrRows consecutive rows of one cache, one wave each (q's
 // int8 limbs in registers).  The cache goes through LDS in chunks of 128 tokens,
@@ -2577,6 +2577,28 @@ static void launch_rescore(const uint8_t* q, const float* qs, const uint8_t* k, 
 #undef MOSAIC_RESCORE
 }
 
+// Where the row kernel runs: on the shortest caches (us, certified path against
+// row kernel, 64 heads, 64 entries: 1 row 18.2 / 12.4, 4096 rows of a cache each
+// 211 / 185, 16384 rows 917 / 746), and where many rows share a short one.  It
+// takes about 0.13 us an entry for each round of 256 workgroups, whatever topk;
+// the certified path's time goes with the rows and grows with topk.  The line is
+// where the row kernel is ahead both with every row at full length and with a
+// prompt's triangular lengths, which the host does not see: entries times rounds
+// up to 13/16 of the rows from 512 picks (all of them where it runs several
+// rounds), 5/8 from 256, 1/2 below (512 picks, full / triangular: 1280 rows over 1024
+// entries 185 -> 135 and 160 -> 133, 512 over 448 62 -> 64 triangular, 1100 over 1100
+// 185 -> 161 but 152 -> 160, 4096 over 2048 639 -> 534 and 546 -> 303, 2560 over 2048
+// 387 -> 528; 64 picks: 1024 over 512 89 -> 70 and 86 -> 69, 1024 over 1024 98 -> 134;
+// 1 pick: 2048 over 1024 154 -> 136 and 142 -> 135, 4096 over 2048 387 -> 530).
+static bool dsa_rows_kernel(int64_t b, int64_t kdiv, int64_t l, int64_t topk) {
+  if (l <= 0 || l > kDrMaxL) return false;
+  if (l <= 64) return true;
+  if (kdiv < kDrRows || b < (l <= 128 ? 256 : 512)) return false;
+  const int64_t rounds = (b / kdiv * ((kdiv + kDrRows - 1) / kDrRows) + 255) / 256;
+  const int64_t sixteenths = topk >= 512 ? (rounds > 1 ? 16 : 13) : topk >= 256 ? 10 : 8;
+  return 16 * l * rounds <= sixteenths * b;
+}
+
 struct MlaWs {
   uint16_t* part_o;
   float* part_ml;
@@ -2658,14 +2680,7 @@ static int indexer_topk_impl(const uint8_t* q, const float* q_s, const uint8_t* 
                    workspace_bytes, need);
   if (b == 0) return kOk;
   hipStream_t st = (hipStream_t)stream;
-  // The row kernel: on the shortest caches, and where many rows share a short
-  // one (us, certified path against row kernel, 64 heads: 1 row of 64 tokens 19.2
-  // / 13.0; 256 rows sharing 128 tokens 28.0 / 24.0, 256 tokens 34.0 / 40.1; 512
-  // rows sharing 256 tokens 52.8 / 40.9, 512 tokens 75.5 / 71.5, 1024 tokens 117 /
-  // 136; 1024 rows sharing 1024 tokens 180 / 140; 4096 rows sharing 1024 tokens
-  // 617 / 281).  A row takes one wave, so few rows over a longer cache, or rows
-  // with a cache each, leave it to the certified path.
-  if (l > 0 && (l <= 64 || (kdiv >= kDrRows && b >= 256 && (l <= 128 || (b >= 512 && l <= b && l <= kDrMaxL))))) {
+  if (dsa_rows_kernel(b, kdiv, l, topk)) {
     const int groups = (int)(b / kdiv);
     const dim3 grid((unsigned)(groups * ((kdiv + kDrRows - 1) / kDrRows)));
 #define MOSAIC_ROWS_TOPK(HT)                                                                                        \

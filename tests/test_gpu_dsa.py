@@ -516,6 +516,33 @@ def test_indexer_rows_kernel_vs_oracle(dev, groups, rows, h, l, cache, topk, tie
         np.testing.assert_array_equal(got[r:r + 1], ref)
 
 
+@pytest.mark.parametrize("rows,per,h,l,topk,one_kernel", [
+    # on either side of the line: below and from 256 and 512 picks, several rounds of workgroups, few rows a cache
+    (512, 512, 16, 256, 1, True), (512, 512, 16, 257, 255, False), (1024, 1024, 16, 640, 256, True),
+    (1024, 1024, 16, 641, 511, False), (640, 640, 64, 513, 512, True), (640, 640, 16, 521, 512, False), (1300, 1300, 16, 1025, 2048, True),
+    (512, 512, 64, 512, 512, False), (4096, 4096, 16, 2048, 700, True), (4096, 4096, 16, 2048, 300, False),
+    (2560, 2560, 16, 2048, 512, False), (520, 8, 32, 129, 512, True), (511, 511, 16, 129, 512, False),
+    (70, 1, 16, 64, 512, True), (70, 1, 16, 65, 512, False)])
+def test_indexer_rows_dispatch(dev, rows, per, h, l, topk, one_kernel):
+    """Where many rows over short caches take the one-kernel path (one launch) and where the certified path
+    (four), with every sort width of the former; sampled rows against the oracle."""
+    from mosaic_amd import _lib, ops
+    rng = np.random.default_rng(rows + l + topk)
+    q, qs = D.quantize_rows_e4m3(rng.standard_normal((rows, h, 128)))
+    k, ks = D.quantize_rows_e4m3(rng.standard_normal((rows // per, l, 128)))
+    w = rng.standard_normal((rows, h)).astype(np.float32)
+    lengths = rng.integers(0, l + 1, rows).astype(np.int32)
+    lengths[0] = l
+    t = _t(dev, q, qs, k, ks, w, lengths)
+    before = _lib.lib().mosaic_launch_count()
+    got = ops.dsa_indexer_topk_shared(*t[:5], topk, t[5]).cpu().numpy()
+    assert _lib.lib().mosaic_launch_count() - before == (1 if one_kernel else 4)
+    for r in sorted({0, rows - 1, *rng.integers(0, rows, 8).tolist()}):
+        g = r // per
+        ref = D.indexer_topk(q[r:r + 1], qs[r:r + 1], k[g:g + 1], ks[g:g + 1], w[r:r + 1], topk, lengths[r:r + 1])
+        np.testing.assert_array_equal(got[r:r + 1], ref)
+
+
 def test_indexer_drop_in_prefill_causal(dev):
     """Indexer scoring at start_pos 0: position i sees the first (i + 1) // 4
     compressed entries, masked picks are -1, valid ones + offset (the query
