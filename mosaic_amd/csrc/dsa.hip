@@ -2632,9 +2632,15 @@ static int mla_head_tiles(int64_t b, int64_t h, int S) {
 // 16.1; below, the block kernel spreads 16-head groups wider: 2 rows of 512 14.7 /
 // 15.4, 64 heads x 4 rows of 512 14.6 / 15.4; above, its fewer partials win: 32
 // rows of 4096 128 / 139).
+//
+// fp32 partials past 320 workgroups (42 MB) cost more than the shorter chain gives
+// where the block kernel's grid is one whole round: 32 rows of 128 heads, 896 picks
+// 45.5 / 47.5, 1000 48.6 / 52.3, but 640 picks 39.2 / 38.9; 24 rows, whose blocks
+// need a second round, 1000 picks 67.3 / 42.5.
 static int mla_chunks(int64_t b, int64_t h, int64_t topk) {
   const int64_t chunks = (topk + kMdTokens - 1) / kMdTokens;
   const int64_t wgs = b * (h / 64) * chunks;
+  if (chunks <= kMdF32Chunks && wgs > 320 && (int64_t)mla_splits(b, topk) * wgs <= 256 * chunks) return 0;
   return h % 64 == 0 && chunks <= 32 && b <= 32 && wgs >= 24 && wgs <= 1024 ? (int)chunks : 0;
 }
 // `chunks`: splits of the whole-split kernel, 0 for the block kernel.  Queries

@@ -49,3 +49,14 @@ def test_fp8_big_tiles_keep_near_ties(m, n, k, kind):
 def test_a8_splits(m, n, k, splits):
     """K slices of the dense A8 GEMM, above the row count where the partials' rate changes and below."""
     assert _lib.lib().mosaic_mxt16_linear_a8_workspace_bytes(m, n, k) == (4 * m * n * splits if splits > 1 else 0)
+
+
+@pytest.mark.parametrize("b,h,topk,whole_splits", [
+    (32, 128, 640, True), (32, 128, 641, False), (32, 128, 1000, False), (32, 128, 1024, False), (32, 128, 2048, True),
+    (31, 128, 1000, True), (24, 128, 1000, True), (32, 64, 1024, True), (16, 256, 1024, True), (16, 128, 1024, True)])
+def test_mla_whole_splits_with_fp32_partials(b, h, topk, whole_splits):
+    """Up to 1024 picks the whole-split kernel's partials are fp32: 32 rows of 128 heads past 640 picks stay
+    on the block kernel, whose partials are all that the workspace then holds."""
+    size = _lib.lib().mosaic_mla_decode_workspace_bytes
+    splits = size(b, 16, topk) // (b * 16 * 1024)  # the block kernel's (16 heads never take whole splits)
+    assert (size(b, h, topk) > b * splits * h * (1024 + 8)) == whole_splits
