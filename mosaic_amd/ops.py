@@ -24,8 +24,13 @@ RECIPES = {"ceil": 0, "floor": 1}
 # GPU work is a few microseconds, so they avoid building Stream and device
 # objects, ctypes wrappers and no-op views (a one-token linear: 9.1 -> 6.3 us a
 # call among others).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # not public: a build may lack it
+
+
 def _stream() -> int:
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None):

@@ -66,3 +66,18 @@ def test_python_wrappers_reject_cpu_tensors():
     with pytest.raises(ValueError, match="GPU tensor"):
         ops.mx_linear_a16(torch.zeros(1, 128, dtype=torch.bfloat16), torch.zeros(16, 64, dtype=torch.uint8),
                           torch.zeros(16, 4, dtype=torch.uint8))
+
+
+def test_stream_without_the_raw_query(monkeypatch):
+    """A torch build without the private stream query: the public Stream object's handle."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from mosaic_amd import ops
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=77))
+    monkeypatch.setattr(ops, "_raw_stream", lambda device: 100 + device)
+    assert ops._stream() == 103
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream() == 77
