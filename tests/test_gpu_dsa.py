@@ -330,6 +330,67 @@ def test_mla_rows_bf16_unaligned_keeps_split_kernel(dev, skew):
     _close(out.float().cpu().numpy(), D.sparse_attn(q, kv, None, idx, 512 ** -0.5, 512, rows))
 
 
+def _same_class(got, ref):
+    """NaN in the same places, the rest close (bf16 outputs of bf16 probabilities, summed in another order)"""
+    got, ref = got.float().cpu().numpy(), ref.float().cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    _close(np.nan_to_num(got), np.nan_to_num(ref))
+
+
+@pytest.mark.parametrize("with_sink", [False, True])
+def test_mla_rows_nonfinite_as_split_kernel(dev, with_sink):
+    """The row kernel against the split kernel (the same rows, 32 a call) without a sink and with ones that are
+    infinite, for NaN in q, a NaN and an infinite cache value among finite picks, and scores beyond fp32's exp."""
+    from mosaic_amd import ops
+    rows, h, n, t = 64, 32, 100, 64
+    rng = np.random.default_rng(21)
+    q = torch.from_numpy(rng.standard_normal((rows, h, 512)).astype(np.float32)).to(dev).to(torch.bfloat16)
+    kv = torch.from_numpy(rng.standard_normal((1, n, 512)).astype(np.float32)).to(dev).to(torch.bfloat16)
+    idx = np.stack([rng.permutation(90)[:t] for _ in range(rows)]).astype(np.int32)
+    kv[0, 97, 5], kv[0, 98, 7], kv[0, 99, 9] = float("nan"), float("inf"), -float("inf")
+    q[0, 3], q[1, 4, 100] = float("nan"), float("nan")
+    q[5] *= 400.0
+    for r, token in ((2, 97), (3, 98), (4, 99)):
+        idx[r, 40] = token
+    sink = None
+    if with_sink:
+        sink = torch.from_numpy(rng.standard_normal(h).astype(np.float32)).to(dev)
+        sink[0], sink[1] = float("inf"), -float("inf")
+    idx = torch.from_numpy(idx).to(dev)
+    got = ops.mla_sparse_decode_bf16(q, kv, idx, 512 ** -0.5, sink)
+    ref = torch.cat([ops.mla_sparse_decode_bf16(q[i:i + 32], kv, idx[i:i + 32], 512 ** -0.5, sink) for i in (0, 32)])
+    assert bool(torch.isnan(got[2]).all()) and not bool(torch.isnan(got[5:]).any())
+    _same_class(got, ref)
+
+
+@pytest.mark.parametrize("b,t", [(12, 1000), (8, 2048)])  # fp32 and bf16 partials
+@pytest.mark.parametrize("with_sink", [False, True])
+def test_mla_whole_splits_nonfinite_as_block_kernel(dev, b, t, with_sink):
+    """The whole-split kernel against the block kernel, which an unaligned q keeps: as above, over an FP8 cache
+    (NaN and infinite scales, NaN and infinite rope values)."""
+    from mosaic_amd import ops
+    h, n = 128, 2200
+    rng = np.random.default_rng(22)
+    q, lat, ls, rope, idx = _mla(rng, b, h, n - 4, t, 64, 0.1)
+    pad = lambda a: np.concatenate([a, a[:, :4]], 1)
+    lat, ls, rope = pad(lat), pad(ls), pad(rope)
+    ls[:, n - 4, 2], ls[:, n - 3, 2] = np.nan, np.inf
+    rope[:, n - 2, 5], rope[:, n - 1, 5] = np.nan, -np.inf
+    q[0, 3], q[1, 4, 100] = np.nan, np.nan
+    q[6] *= 400.0
+    for r in range(4):
+        idx[r + 2, 40] = n - 4 + r
+    _, latd, lsd, rd, idxd = _t(dev, q, lat, ls, rope, idx)
+    qd, qs, rd = torch.from_numpy(q).to(dev).to(torch.bfloat16), _skewed(q, dev), rd.to(torch.bfloat16)
+    sink = None
+    if with_sink:
+        sink = torch.from_numpy(rng.standard_normal(h).astype(np.float32)).to(dev)
+        sink[0], sink[1] = float("inf"), -float("inf")
+    got, ref = (ops.mla_sparse_decode(x, latd, lsd, rd, idxd, 0.06, sink) for x in (qd, qs))
+    assert not torch.equal(got, ref) and not bool(torch.isnan(got[6:]).any())
+    _same_class(got, ref)
+
+
 def test_mla_wide_score_range(dev):
     """Scores rising by over a hundred nats along the token order (the rope part
     grows 300-fold): every head's running maximum moves past the lazy margin
@@ -491,9 +552,9 @@ def test_indexer_drop_in_decode(dev):
     (1, 256, 64, 128, 128, 100, 1), (2, 514, 64, 129, 129, 64, 0), (1, 600, 64, 300, 333, 512, 1),
     (1, 520, 64, 513, 520, 512, 0), (1, 1030, 16, 1025, 1025, 2048, 1), (1, 2048, 16, 2048, 2048, 700, 1)])
 def test_indexer_rows_kernel_vs_oracle(dev, groups, rows, h, l, cache, topk, ties):
-    """Rows over short caches in one kernel: every sort width, batches of 16 and chunks of 128 tokens cut
-    short, workgroups with idle waves, caches longer than l, lengths below 0, past l and 0, equal scores,
-    and NaN scores (lowest)."""
+    """Rows over short caches, most in one kernel (the longest per row take the certified path, see
+    test_indexer_rows_dispatch): batches of 16 and chunks of 128 tokens cut short, workgroups with idle waves,
+    caches longer than l, lengths below 0, past l and 0, equal scores, and NaN scores (lowest)."""
     from mosaic_amd import ops
     rng = np.random.default_rng(rows + l)
     q, qs = D.quantize_rows_e4m3(rng.standard_normal((rows, h, 128)))

@@ -60,3 +60,15 @@ def test_mla_whole_splits_with_fp32_partials(b, h, topk, whole_splits):
     size = _lib.lib().mosaic_mla_decode_workspace_bytes
     splits = size(b, 16, topk) // (b * 16 * 1024)  # the block kernel's (16 heads never take whole splits)
     assert (size(b, h, topk) > b * splits * h * (1024 + 8)) == whole_splits
+
+
+def test_fp8_planned_slices_are_never_empty():
+    """Slices are ceil(K blocks / S) blocks each: every S that a plan names fills all of them (33 blocks in 8
+    slices of 5 would leave the eighth starting past K)."""
+    for m in (65, 96, 128, 129, 200, 256, 300, 777, 2048):
+        for n in (16, 128, 512, 577, 1536, 4096, 7168, 18432):
+            for nkb in range(1, 131):
+                kind, splits = _fp8(m, n, 128 * nkb)
+                if kind in (T128, T256):
+                    per = -(-nkb // splits)
+                    assert -(-nkb // per) == splits, (m, n, nkb, splits)
