@@ -131,7 +131,7 @@ int mosaic_mxt16_linear_a16(const uint16_t* x, const uint8_t* packed_t, const ui
 int mosaic_mxt16_linear_a8(const uint8_t* xq, const float* sa, const uint8_t* packed_t, const uint8_t* scale_t,
                            uint16_t* y, int64_t m, int64_t n, int64_t k, void* stream);
 /* Scratch bytes of mosaic_mxt16_linear_a8_ws: the fp32 partials of the split-K
- * plan (shapes whose tiles cover at most half of the GPU), else 0. */
+ * plan where the time estimate picks one, else 0. */
 size_t mosaic_mxt16_linear_a8_workspace_bytes(int64_t m, int64_t n, int64_t k);
 /* mosaic_mxt16_linear_a8 with a caller workspace for the split-K plan (without
  * one, or with too few bytes, the shape runs unsplit).  Same replacement as
@@ -153,8 +153,8 @@ int mosaic_fp8_block_gemm(const uint8_t* a, const float* a_s, const uint8_t* b, 
                           int out_dtype, int64_t m, int64_t n, int64_t k, void* stream);
 
 /* Bytes of the fp32 partials workspace that mosaic_fp8_block_gemm_ws uses to
- * split K over up to 8 slices when the output tiles cover fewer than half of
- * the GPU (0: the shape is not split).  No counterpart in the reference, whose
+ * split K over up to 8 slices where its time estimate says so (0: the shape is
+ * not split).  No counterpart in the reference, whose
  * fp8_gemm launches allocate nothing; it serves the same call sites. */
 size_t mosaic_fp8_block_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 
@@ -357,7 +357,8 @@ int mosaic_moe_a8_forward(const uint16_t* x, const float* logits, int32_t* ids, 
                           void* workspace, size_t workspace_bytes, void* const* stage_events, void* stream);
 
 /* ----------------------------------------------------------- DSA decode -- */
-/* Workspace bytes of mosaic_dsa_indexer_topk for b rows of l cached tokens. */
+/* Workspace bytes of mosaic_dsa_indexer_topk for b rows of l cached tokens
+ * (also asked of calls over short caches, whose one-kernel path leaves it unused). */
 size_t mosaic_dsa_indexer_workspace_bytes(int64_t b, int64_t l);
 
 /* FP8 lightning indexer + top-k, replacing Indexer.forward's scoring and topk
@@ -414,7 +415,10 @@ int mosaic_dsa_head_attention(const uint16_t* q, const uint16_t* k, const uint16
                               int64_t h, int64_t ctx, int64_t d, int64_t dv, int64_t topk, float scale,
                               void* workspace, size_t workspace_bytes, void* stream);
 
-/* Workspace bytes of mosaic_mla_sparse_decode. */
+/* Workspace bytes of mosaic_mla_sparse_decode and its bf16 form: room for the
+ * partials of whichever split kernel the call may take.  A call with room for
+ * the block kernel's only is taken and runs that one; calls of 64 and more rows
+ * over 512-wide bf16 caches are checked for it too, but leave it unused. */
 size_t mosaic_mla_decode_workspace_bytes(int64_t b, int64_t h, int64_t topk);
 
 /* MLA decode over the selected KV entries, replacing sparse_attn

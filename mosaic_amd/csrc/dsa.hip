@@ -1676,9 +1676,11 @@ struct MlaPart<float> {
 // kernel's many small ones (512 picks, relative error against 64 bits: 2.4e-3 on
 // the block kernel, 2.5e-3 with bf16 partials here).  q goes through LDS first (its
 // fragments straight from memory cost 36 scattered loads a wave, 8 us of the
-// chain).  Measured: 8 rows x 128 heads x 2048 picks 27.9 us on the block kernel,
-// ~17 here; what is left is the chain itself (~24,000 cycles: ids and q 9,000,
-// conversion 4,000, scores 3,400, softmax 2,300, values 2,700, stores 1,800).
+// chain).  Measured, 8 rows x 128 heads x 2048 picks: the whole call 32.1 -> 22.4
+// us, of which this kernel takes 17.1 in a kernel trace and the combine 7.1; what is
+// left is the chain itself (about 24,000 cycles by timestamps in a scratch build:
+// ids and q 9,000, conversion 4,000, scores 3,400, softmax 2,300, values 2,700,
+// stores 1,800).
 constexpr int kMdTokens = 128;
 constexpr int kMdF32Chunks = 8;      // up to this many splits store fp32 partials
 constexpr int kMdRow = kMlaDl + 8;   // bf16 per latent row in LDS
@@ -1728,8 +1730,10 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
   }
   // Wave wv gathers tokens 16 i + 2 wv + {0, 1}: latent piece i is token 2 wv +
   // lane / 32 of the i-th 16, bytes 16 (lane % 32); rope piece j covers eight of
-  // the tokens, 8 values at 8 (lane % 8).  The ids are wave-uniform, so they come
-  // by scalar loads, which do not wait for q's copies.
+  // the tokens, 8 values at 8 (lane % 8).  The ids are wave-uniform and come by
+  // scalar loads.  (The choice between a half-wave's two ids compiles to private
+  // memory, 80 bytes a lane, whose loads come back behind q's copies: the gather's
+  // addresses wait for q, a part of the 9,000 cycles above.)
   const int32_t* ids = idx + (int64_t)b * topk + t0;
   const int lp = lane & 31, rp = lane & 7, lt = 2 * wv + (lane >> 5);
   int id2[kMdLat][2];
@@ -1737,7 +1741,7 @@ __global__ void __launch_bounds__(512) mla_decode_chunk_kernel(const uint16_t* _
   for (int i = 0; i < kMdLat; ++i)
 #pragma unroll
     for (int u = 0; u < 2; ++u) id2[i][u] = ids[min(16 * i + 2 * wv + u, nt - 1)];
-  __builtin_amdgcn_sched_barrier(0);  // all loads first: one wait instead of sixteen
+  __builtin_amdgcn_sched_barrier(0);  // the loads first: a wait for eight of them at a time
 #pragma unroll
   for (int i = 0; i < kMdLat; ++i)
 #pragma unroll
@@ -2063,8 +2067,10 @@ __global__ void __launch_bounds__(256) mla_combine_tiles_kernel(const TP* __rest
 //
 // Bound by the chains of a period (scoring: 32 MFMAs on LDS operands, then the
 // softmax; value: copies, then 32 MFMAs) and by the gather, 32 KB a block and
-// CU: 2048 rows x 64 heads x 512 with 128 + up to 512 picks 686 -> 185 us
-// (550 TFLOP/s on the valid picks), of which copies alone take ~100.
+// CU: a call of 2048 rows x 64 heads x 512 with 128 + up to 512 picks 666 -> 178 us
+// (570 TFLOP/s on the valid picks), of which copies alone take ~100.  All 256
+// registers are taken and 9 spill: the scoring waves reload them between the pick
+// loads at an item's start.
 constexpr int kMrStages = 4;
 constexpr int kMrRow = kMlaDl * 2 + 16;  // bytes per staged row
 constexpr int kMrStage = kMlaBT * kMrRow;

@@ -516,8 +516,10 @@ __global__ void __launch_bounds__(BM * kTileN / kTileWN, 1) fp8_gemm_tiled_kerne
 }
 
 // C = sum over the S (at most 8) slices of part, in slice order; 4 elements per
-// thread.  Where rows of 4 stay aligned (VEC) every slice's 16 bytes are loaded
-// before the sum.
+// thread, 16 bytes a slice where rows of 4 stay aligned (VEC).  S is a run-time
+// count, so the compiled loads keep a branch and a wait each and the slices arrive
+// one after another (196 registers; 7.0 us for 4 slices of 128 x 7168, 18.4 MB,
+// in the kernel trace).
 template <bool VEC>
 __global__ void __launch_bounds__(256) fp8_splitk_reduce_kernel(const float* __restrict__ part, int S, int64_t mn,
                                                                 void* __restrict__ C, int out_f32) {
@@ -811,7 +813,7 @@ static void launch_fp8_mid(const uint8_t* a, const float* as, const uint8_t* b, 
   if (S > 1) launch_fp8_reduce(part, S, m * n, c, out_f32, st);
 }
 
-// Large tiled kernel (enough 256 x 256 tiles to fill the chip): a workgroup
+// Large tiled kernel (where its estimate is least, see fp8_plan): a workgroup
 // of 8 waves owns a 256 x 256 block of C; wave w owns rows 128 (w >> 2) and
 // columns 64 (w & 3) of it.  Twice the columns of the 256 x 128 kernel for
 // the same A block: 256 instead of 171 flops per byte copied into LDS.  A
@@ -1075,9 +1077,9 @@ extern "C" int mosaic_fp8_block_dequant(const uint8_t* w, const float* s, uint16
 // Kernel choice of the block GEMM.  kind 0: skinny, 1: tiled<128>, 2: tiled<256>,
 // 3: big tiles, 4: decode ring (M <= 16 with N >= 4096, or narrower N when K has
 // at least 32 blocks), 5: mid kernel (17..64 rows, N % 16 == 0, its own K split;
-// and 12..16 rows where fp8_mid_small holds).  The tiled kernels split K into S slices (S > 1 needs the
-// S * M * N * 4-byte partials workspace) when their tiles cover fewer than
-// half of the 256 CUs: S = min(8, 256 / tiles, K-blocks / 4).
+// and 12..16 rows where fp8_mid_small holds).  The tiled kernels split K into up
+// to 8 slices of at least 4 blocks (S > 1 needs the S * M * N * 4-byte partials
+// workspace) where the estimate below says so.
 struct Fp8Plan {
   int kind, S;
 };
@@ -1095,8 +1097,8 @@ struct Fp8Plan {
 // K block, 128 0.71, 144 1.08, 192 1.05).  One step for all row counts split 200 x
 // 18432 x 7168 three ways at 73.9 us where the whole K takes 64.1 (205 x 21584 x
 // 11264 106.8 / 99.8, 171 x 23312 x 15232 150.1 / 138.4), and left 245 x 11680 x
-// 10112 on 128-row tiles (66.7 / 61.8); of 14 shapes whose plan moved, 136 x 5696 x
-// 6656 alone lost (25.7 / 26.1).
+// 10112 on 128-row tiles (66.7 / 61.8); of 14 shapes that this moved, 136 x 5696 x
+// 6656 alone lost (25.7 / 26.1; 30.9 by the tile counts).
 static float fp8_tiled_time(int kind, int S, int64_t m, int64_t n, int64_t k) {
   const int64_t bm = kind == 1 ? 128 : 256, bn = kind == 3 ? 256 : 128, nkb = k / 128;
   const int64_t steps = (nkb + S - 1) / S, slices = (nkb + steps - 1) / steps, n_row = (m + bm - 1) / bm;
